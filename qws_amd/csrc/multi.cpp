@@ -116,6 +116,7 @@ void Fused::prec(std::vector<PrecJob>& jobs, bool ddd, int nsap, int nm, SapFusi
   for (const PrecJob& j : jobs) {
     const Lattice& L = *j.L;
     fuse = fuse && L.fused_ok<float>() && L.use_fb_ && sap_face_buffer_floats(L.g_) > 0 && L.g_.Vb == L0.g_.Vb &&
+           sap_is_4444(L.g_) == sap_is_4444(L0.g_) &&  // one kernel for all, the one each runs alone
            L.nl32_ == L0.nl32_ && L.st_ == L0.st_ && L.st_ == fz->stream() && (j.upd != nullptr) == (jobs[0].upd != nullptr);
   }
   if (!fuse) {
@@ -178,6 +179,7 @@ void Fused::prec(std::vector<PrecJob>& jobs, bool ddd, int nsap, int nm, SapFusi
     m.table = table[s0.colour];
     m.n = ntab[s0.colour];
     m.xcd = L0.g_.xcd_remap;
+    m.b4 = sap_is_4444(L0.g_);
     Rec r;
     std::memset(&r, 0, sizeof(r));
     r.m = m, r.flags = s0.flags | (s0.pupd ? SAP_SRC_PUPD : 0), r.face = s0.face ? 1 : 0;

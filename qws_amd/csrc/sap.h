@@ -48,16 +48,20 @@ template <typename S> struct SapPart {
   SapSrcUpdate upd;
 };
 // A launch fused over several lattices: workgroup w runs block table[w].y of part
-// table[w].x (device arrays).  The parts share the block volume, the link storage,
-// the flags and nm; xcd: map the workgroups to the table XCD by XCD.
+// table[w].x (device arrays).  The parts share the block volume (and whether the blocks
+// are 4^4), the link storage, the flags and nm; xcd: map the workgroups to the table XCD by XCD.
 template <typename S> struct SapMulti {
   const SapPart<S>* parts = nullptr;
   const int2* table = nullptr;
   int n = 0;
   int xcd = 1;
+  int b4 = 0;        // 1: every part has 4^4 blocks (sap4.hip), 0: none has
+  int reserved = 0;  // no padding: launch records are compared by their bytes
 };
 
 bool sap_fusable(const Geo& g);
+// 4^4 blocks: the FP32 kernel of sap4.hip
+bool sap_is_4444(const Geo& g);
 // floats per RHS of the face buffer, or 0 when the block shape does not allow it
 // (its slots must fit the iterate's LDS: 2 sum_mu Vb / B_mu <= 2 Vb)
 long long sap_face_buffer_floats(const Geo& g);
@@ -72,6 +76,11 @@ void launch_sap_block(const Geo& g, BlockSel sel, const Batch& B, int nl, float 
 // The same over several lattices in one launch (FP32 storage): vb = their sites per
 // block, nl their FP32 link storage; every part has a face buffer when `flags` use one.
 void launch_sap_multi(const SapMulti<float>& m, int vb, int nl, int nm, int flags, hipStream_t st);
+// launch_sap_block<float> and launch_sap_multi on 4^4 blocks (sap4.hip)
+void launch_sap_4444(const Geo& g, BlockSel sel, const Batch& B, int nl, float kappa, int nm, int flags, float* s,
+                     const float* in, const float* qface, float* qout, float* out, const float* U, const float* C,
+                     float* fb, long long fbs, hipStream_t st, const SapSrcUpdate& upd);
+void launch_sap_4444_multi(const SapMulti<float>& m, int nl, int nm, int flags, hipStream_t st);
 // launch_sap_face over several lattices (part.out, .fb, .fbs, .U, .C; factor in .kappa)
 void launch_sap_face_multi(const SapMulti<float>& m, int vb, int nl, hipStream_t st);
 

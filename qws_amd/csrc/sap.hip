@@ -17,8 +17,16 @@
 
 #include "kernels.h"
 #include "sap.h"
+#include "sap_device.h"
 
 namespace qws {
+
+// a launch that reads or writes the face buffer takes no gathers; a face update that
+// reads the buffer is always preceded by a launch that wrote it
+static void check_face_flags(int flags) {
+  if ((flags & SAP_FACE_PRO) && (flags & SAP_FACE_OUT) && !(flags & SAP_FACE_FB))
+    throw std::invalid_argument("fused SAP: a face update in a face-buffer launch must read the buffer");
+}
 
 namespace sap256 {
 constexpr int VB = 256;  // 4^4 blocks
@@ -51,6 +59,13 @@ void launch_sap_block(const Geo& g, BlockSel sel, const Batch& B, int nl, float 
         (const void*)upd.p != (const void*)in)
       throw std::invalid_argument("fused SAP: the source update needs FP32, SAP_SRC_IN and in == p, r, q, scalars");
   }
+  if constexpr (std::is_same<S, float>::value) {
+    if (sap_is_4444(g)) {
+      check_face_flags(flags);
+      launch_sap_4444(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);
+      return;
+    }
+  }
   if (g.Vb == 512) sap512::launch<S>(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);
   else sap256::launch<S>(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);
 }
@@ -68,6 +83,11 @@ void launch_sap_multi(const SapMulti<float>& m, int vb, int nl, int nm, int flag
   if (nm < 1) nm = 1;  // the first application is unconditional (static_solver.cc:77-101)
   if (flags & SAP_SRC_PUPD) {
     if (!(flags & SAP_SRC_IN)) throw std::invalid_argument("fused SAP: the source update needs SAP_SRC_IN");
+  }
+  if (m.b4) {
+    check_face_flags(flags);
+    launch_sap_4444_multi(m, nl, nm, flags, st);
+    return;
   }
   if (vb == 512) sap512::launch_multi(m, nl, nm, flags, st);
   else if (vb == 256) sap256::launch_multi(m, nl, nm, flags, st);

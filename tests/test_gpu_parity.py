@@ -212,6 +212,47 @@ def test_fused_sap_face_buffer_is_bitwise_the_gather(L, B, su3, nsap, nm):
     assert rel(res[True][0], p.orc.prec_ddd_s(srcs[0], nsap, nm)) < 5e-6
 
 
+@pytest.mark.parametrize("su3", [True, False])
+@pytest.mark.parametrize("L,nsap,nm", [([8, 8, 8, 8], 1, 1), ([8, 8, 8, 8], 3, 2), ([24, 8, 16, 8], 2, 1),
+                                       ([24, 8, 16, 8], 0, 5), ([32, 16, 32, 32], 1, 2)])
+def test_fused_sap_4444(L, nsap, nm, su3):
+    """The FP32 kernel for 4^4 blocks (hops by link, not by site) where both neighbours
+    of a block are the same one, at extents that differ in every direction, with one Jacobi
+    step, with 12- and 18-real links, and on 1024 blocks per colour (second workgroups
+    start late): the oracle's result, by the face buffer bit for bit as by gathers.  On the
+    largest lattice against the step-by-step kernels.  FP32 rounding: 1e-6 at most over
+    the few hundred operations behind a component, 5e-6 allowed as in the tests above."""
+    big = np.prod(L) > 100000
+    if big:
+        lat = Q.Lattice(L, [4, 4, 4, 4], -1, 12 if su3 else 18, kappa=0.125)
+        lat.generate_gauge(0.3, 1)
+        lat.compute_clover(1.0)
+        bs = np.random.default_rng(11).standard_normal((lat.V, 3, 4, 2)).astype(np.float32)
+    else:
+        p = Problem(L, [4, 4, 4, 4], kappa=0.125, seed=10, su3=su3)
+        lat, bs = p.lat, p.b.astype(np.float32)
+    inp = lat.spinor(Q.F32, bs)
+
+    def both():
+        o1, o2 = lat.spinor(Q.F32), lat.spinor(Q.F32)
+        lat.prec_ddd(o1, inp, nsap, nm)
+        lat.prec_s(o2, inp, nsap, nm)
+        return o1.download(), o2.download()
+
+    got = both()
+    lat.set_sap_face_buffer(False)
+    for a, b in zip(got, both()):
+        assert np.array_equal(a, b)
+    lat.set_sap_face_buffer(True)
+    if big:
+        lat.set_sap_fused(False)
+        want = both()
+    else:
+        want = p.orc.prec_ddd_s(bs, nsap, nm), p.orc.prec_s(bs, nsap, nm)
+    for a, b in zip(got, want):
+        assert rel(a, b) < 5e-6
+
+
 @pytest.mark.skipif(not RW.available(), reason="oracle/_ref/libqws_ref.so not built")
 def test_dropin_plain_dd_solvers_and_helpers_case0():
     """bicgstab_dd_s_/bicgstab_dd_d_ (plain BiCGStab on D) through the QWS ABI on
