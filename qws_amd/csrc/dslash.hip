@@ -252,25 +252,15 @@ k_dslash_lds_d(Geo g, const int* __restrict__ order, const int* __restrict__ act
   }
 }
 
-template <typename S>
-__global__ void __launch_bounds__(HOP_THREADS)
-k_zero_blocks(Geo g, const int* list, int wg_per_blk, int nrhs, long long stride, const int* active, S* out) {
-  using R = typename Store<S>::R;
-  const int bi = blockIdx.x / wg_per_blk;
-  const int blk = list ? list[bi] : bi;
-  const int loc = (blockIdx.x - bi * wg_per_blk) * HOP_THREADS + threadIdx.x;
-  if (loc >= g.Vb) return;
-  const long long s = (long long)blk * g.Vb + loc;
-  Cx<R> v[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) v[k] = {0, 0};
-  for (int r = 0; r < nrhs; ++r)
-    if (!active || active[r]) SpinorIO<S>::store(out + r * stride, s, g.V, v);
-}
-
 template <typename S, int NL>
 void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a,
                 const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st) {
+  if (split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value)) {
+    SplitPart<S> p;
+    p.sel = sel, p.set = set, p.gamma = gamma, p.out = out, p.a = a, p.b = b, p.c = c, p.in = in;
+    launch_split<S, NL>(g, p, SplitPart<S>(), B, U, C, st);
+    return;
+  }
   if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
     // the full operator: one lean launch per right-hand side
     if constexpr (std::is_same<S, float>::value) {
@@ -321,13 +311,6 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
 #undef HOP_ARGS
 }
 
-template <typename S>
-void launch_zero_blocks(const Geo& g, BlockSel sel, const Batch& B, S* out, hipStream_t st) {
-  const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
-  hipLaunchKernelGGL((k_zero_blocks<S>), dim3(sel.n * wpb), dim3(HOP_THREADS), 0, st, g, sel.list, wpb, B.n, B.stride,
-                     B.active, out);
-}
-
 #define INST_HOP(S, NL)                                                                                           \
   template void launch_hop<S, NL>(const Geo&, BlockSel, const Batch&, int, typename Store<S>::R, S*, const S*,     \
                                   const S*, const S*, const S*, const S*, const S*, hipStream_t);
@@ -336,8 +319,5 @@ INST_HOP(float, 12)
 INST_HOP(double, 18)
 INST_HOP(__half, 18)
 INST_HOP(__half, 12)
-template void launch_zero_blocks<float>(const Geo&, BlockSel, const Batch&, float*, hipStream_t);
-template void launch_zero_blocks<double>(const Geo&, BlockSel, const Batch&, double*, hipStream_t);
-template void launch_zero_blocks<__half>(const Geo&, BlockSel, const Batch&, __half*, hipStream_t);
 
 }  // namespace qws

@@ -23,9 +23,25 @@ template <typename S, int NL>
 void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a,
                 const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st);
 
-// out = 0 on the selected blocks
-template <typename S>
-void launch_zero_blocks(const Geo& g, BlockSel sel, const Batch& B, S* out, hipStream_t st);
+// One operator of launch_split: the arguments of launch_hop (a face hop set with out == a
+// alone leaves the sites without a face hop untouched) and the hops it may take, all or
+// the faces of some directions: bit 2 mu + (dir < 0), as in Geo.
+template <typename S> struct SplitPart {
+  BlockSel sel = {nullptr, 0};
+  int set = 0;
+  int mask = 0xFF;
+  typename Store<S>::R gamma = 0;
+  S* out = nullptr;
+  const S *a = nullptr, *b = nullptr, *c = nullptr, *in = nullptr;
+};
+// launch_hop's operators (not HOPS_NONE) on one or two block selections in one launch
+// (split.hip): the parts must not write what the other one reads.  Vb < 2^20, V < 2^28.
+template <typename S, int NL>
+void launch_split(const Geo& g, const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B, const S* U, const S* C,
+                  hipStream_t st);
+
+// Whether launch_split is the faster one for the hop set on that many sites (split.hip).
+bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64);
 
 // ---- BiCGStab vector kernels (full lattice, n = number of complex numbers)
 struct Scalars {

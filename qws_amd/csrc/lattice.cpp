@@ -445,6 +445,36 @@ void Lattice::hop(BlockSel s, const Batch& B, int set, typename Store<S>::R gamm
     launch_hop<S, 12>(g_, s, B, set, gamma, out, a, b, c, in, f.U, f.C, st_);
 }
 
+// Two operators that do not depend on each other: one launch where few sites are at work.
+template <typename S> void Lattice::hop2(const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B) {
+  const FieldSet<S> f = fields<S>();
+  // (a pair is worth it to twice the limit of face hops alone: 32 16^3 by halves, FP32 12.6 + 13.6 us and a launch less)
+  if (split_pays(g_, HOPS_FACE, (p0.sel.n + p1.sel.n) * g_.Vb / (p1.sel.n ? 2 : 1), B.n, sizeof(S) == 8)) {
+    if (f.nl == 18) launch_split<S, 18>(g_, p0, p1, B, f.U, f.C, st_);
+    else if constexpr (!std::is_same<S, double>::value) launch_split<S, 12>(g_, p0, p1, B, f.U, f.C, st_);
+    return;
+  }
+  for (const SplitPart<S>* p : {&p0, &p1}) {
+    if (p->sel.n == 0) continue;
+    Geo g = g_;
+    g.hopmask &= p->mask;
+    if (f.nl == 18) launch_hop<S, 18>(g, p->sel, B, p->set, p->gamma, p->out, p->a, p->b, p->c, p->in, f.U, f.C, st_);
+    else if constexpr (!std::is_same<S, double>::value)
+      launch_hop<S, 12>(g, p->sel, B, p->set, p->gamma, p->out, p->a, p->b, p->c, p->in, f.U, f.C, st_);
+  }
+}
+
+// s_c += kappa T^-1 H_face q with s_c read from `src` (where it is not s itself, every
+// site is written).  zero_own: q counts as zero on the blocks of colour c (improper
+// colouring: the directions in which a block is its own neighbour).
+template <typename S> SplitPart<S> Lattice::face_part(int c, S* s, const S* src, const S* q, bool zero_own) const {
+  SplitPart<S> p;
+  p.sel = sel(c), p.set = HOPS_FACE, p.gamma = (typename Store<S>::R)kappa_, p.out = s, p.a = src, p.in = q;
+  for (int m = 0; m < 4; ++m)
+    if (zero_own && g_.NB[m] == 1) p.mask &= ~(3 << (2 * m));
+  return p;
+}
+
 #define DISPATCH_PREC(prec, CALL)                                  \
   do {                                                             \
     if ((prec) == P64) { using S = double; CALL; }                 \
@@ -497,16 +527,19 @@ void Lattice::jinv(int prec, void* x, const void* b, int colour, int nm) {
 //   q_c = A_c s_c ;  s_c += in_c - D_in q_c ;  s_o += kappa T^-1 H_face q
 template <typename S>
 void Lattice::sap_sweeps(const Batch& B, const S* in, S* s, S* q, S* tmp, int nsap, int nm) {
-  using R = typename Store<S>::R;
-  const R k = (R)kappa_;
-  const int pr = sizeof(S) == 8 ? P64 : sizeof(S) == 4 ? P32 : P16;
-  QWS_HIP(hipMemcpyAsync(s, in, spinor_bytes(pr) * B.n, hipMemcpyDeviceToDevice, st_));
-  if (improper_) launch_zero_blocks<S>(g_, sel(1), B, q, st_);
+  if (nsap == 0) {
+    const int pr = sizeof(S) == 8 ? P64 : sizeof(S) == 4 ? P32 : P16;
+    QWS_HIP(hipMemcpyAsync(s, in, spinor_bytes(pr) * B.n, hipMemcpyDeviceToDevice, st_));
+  }
+  const S* src = in;  // s = in, read in place by the half-sweep that first writes s
   for (int isap = 0; isap < nsap; ++isap)
     for (int c = 0; c < 2; ++c) {
-      jinv_t<S>(B, c, q, s, tmp, nm);
-      hop<S>(sel(c), B, HOPS_INSIDE, k, s, s, in, q, q);  // s_c = s_c + in_c - q_c + kappa T^-1 H_in q_c
-      hop<S>(sel(1 - c), B, HOPS_FACE, k, s, s, nullptr, nullptr, q);
+      jinv_t<S>(B, c, q, src, tmp, nm);
+      SplitPart<S> p;  // s_c = s_c + in_c - q_c + kappa T^-1 H_in q_c
+      p.sel = sel(c), p.set = HOPS_INSIDE, p.gamma = (typename Store<S>::R)kappa_;
+      p.out = s, p.a = src, p.b = in, p.c = q, p.in = q;
+      hop2<S>(p, face_part<S>(1 - c, s, src, q, isap == 0 && c == 0), B);  // q_1 = 0 before its first solve
+      src = s;
     }
 }
 
@@ -640,22 +673,10 @@ void Lattice::prec_ddd_t(const Batch& B, S* out, const S* in, int nsap, int nm, 
   if (upd && !std::is_same<S, float>::value) throw std::logic_error("prec_ddd_t: the direction update is FP32");
   S* tmp = (S*)work("sap_tmp", spinor_bytes(pr) * B.n);
   sap_sweeps<S>(B, in, s, q, tmp, nsap, nm);
-  if (improper_) launch_zero_blocks<S>(g_, sel(1), B, q, st_);
   jinv_t<S>(B, 0, q, s, tmp, nm);
-  hop<S>(sel(0), B, HOPS_INSIDE, -k, out, q, nullptr, nullptr, q);  // out_e = D_in q_e
-  if (improper_) {
-    hop<S>(sel(1), B, HOPS_FACE, k, s, s, nullptr, nullptr, q);      // s_o -= D_face q (q_o = 0)
-    jinv_t<S>(B, 1, q, s, tmp, nm);
-    hop<S>(sel(1), B, HOPS_INSIDE, -k, out, q, nullptr, nullptr, q);  // out_o = D_in q_o
-    hop<S>(sel(0), B, HOPS_FACE, -k, out, out, nullptr, nullptr, q);  // out_e += D_face q
-    hop<S>(sel(1), B, HOPS_FACE, -k, out, out, nullptr, nullptr, q);  // out_o += D_face q
-  } else {
-    hop<S>(sel(1), B, HOPS_FACE, -k, out, nullptr, nullptr, nullptr, q);  // out_o = D_oe q_e
-    hop<S>(sel(1), B, HOPS_FACE, k, s, s, nullptr, nullptr, q);           // s_o -= out_o
-    jinv_t<S>(B, 1, q, s, tmp, nm);
-    hop<S>(sel(1), B, HOPS_INSIDE, -k, out, out, q, nullptr, q);          // out_o += D_in q_o
-    hop<S>(sel(0), B, HOPS_FACE, -k, out, out, nullptr, nullptr, q);      // out_e += D_eo q_o
-  }
+  hop2<S>(face_part<S>(1, s, s, q, true), SplitPart<S>(), B);  // s_o -= D_face q (q_o = 0)
+  jinv_t<S>(B, 1, q, s, tmp, nm);
+  hop<S>(sel(-1), B, HOPS_ALL, -k, out, q, nullptr, nullptr, q);  // out = D q, both colours in one pass
 }
 
 // prec_s_ (qws.cc:929-975): out = M_SAP in
@@ -690,9 +711,8 @@ void Lattice::prec_s_t(const Batch& B, S* out, const S* in, int nsap, int nm) {
   }
   S* tmp = (S*)work("sap_tmp", spinor_bytes(pr) * B.n);
   sap_sweeps<S>(B, in, s, q, tmp, nsap, nm);
-  if (improper_) launch_zero_blocks<S>(g_, sel(1), B, out, st_);
   jinv_t<S>(B, 0, out, s, tmp, nm);
-  hop<S>(sel(1), B, HOPS_FACE, (R)kappa_, s, s, nullptr, nullptr, out);
+  hop2<S>(face_part<S>(1, s, s, out, true), SplitPart<S>(), B);
   jinv_t<S>(B, 1, out, s, tmp, nm);
 }
 

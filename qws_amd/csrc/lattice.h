@@ -294,6 +294,8 @@ class Lattice {
   template <typename S>
   void hop(BlockSel s, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a, const S* b,
            const S* c, const S* in);
+  template <typename S> void hop2(const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B);
+  template <typename S> SplitPart<S> face_part(int c, S* s, const S* src, const S* q, bool zero_own) const;
   template <typename S> void jinv_t(const Batch& B, int colour, S* x, const S* b, S* tmp, int nm);
   template <typename S> void sap_sweeps(const Batch& B, const S* in, S* s, S* q, S* tmp, int nsap, int nm);
   template <typename S> bool fused_ok() const;

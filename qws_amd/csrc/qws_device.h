@@ -39,7 +39,7 @@ struct Geo {
   int nblk;       // number of blocks
   long long V;    // sites
   int tbc;        // +1 periodic / -1 antiperiodic in t
-  int hopmask;    // bit 2*mu + (dir < 0): hop taken by the full operator (0xFF); being a
+  int hopmask;    // bit 2*mu + (dir < 0): hop (face hop in HOPS_FACE) taken, 0xFF for all; being a
                   // runtime value it keeps each hop in its own basic block, so the
                   // compiler cannot hoist all eight neighbour loads (256 -> ~146 VGPRs)
   int xcd_remap;  // 1: map workgroups to blocks XCD by XCD (xcd_remap), 0: identity
@@ -441,7 +441,7 @@ __device__ __forceinline__ void one_hop(const Geo& g, long long s, const SiteC& 
   bool inside;
   long long n = neighbour(g, s, c, MU, DIR, inside);
   if (!take_hop<SET>(inside)) return;
-  if (SET == HOPS_ALL && !(g.hopmask & (1 << (2 * MU + (DIR > 0 ? 0 : 1))))) return;
+  if (SET != HOPS_INSIDE && !(g.hopmask & (1 << (2 * MU + (DIR > 0 ? 0 : 1))))) return;
   Cx<R> v[12], a[6], b[6], u[9];
   SpinorIO<S>::load(in, n, g.V, v);
   project<R, MU, DIR>(v, a);

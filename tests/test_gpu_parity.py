@@ -119,6 +119,53 @@ def test_dslash_kernel_variants(su3):
     p.lat.set_dslash_order(0)
 
 
+@pytest.mark.parametrize("L,B,su3", [([6, 3, 5, 7], [3, 3, 5, 7], False), ([4, 8, 4, 4], [2, 8, 2, 4], True),
+                                     ([32, 10, 9, 23], [16, 10, 9, 23], False), ([16, 16, 32, 40], [4, 4, 4, 4], True)])
+def test_operators_around_the_split_rule(L, B, su3):
+    """The operators with four waves per 64 sites and the ones with a thread per site, on
+    either side of the sizes where one takes over: blocks with a ragged last group of 64
+    sites (105, 64, 33120 sites), whole operators of 1036 groups next to their halves of
+    518, and 5120 groups of 4^4 blocks, where every staged kernel is the general one's
+    equal bit for bit.  D against the oracle, and D = D_in + D_face on each colour."""
+    p = Problem(L, B, kappa=0.125, seed=14, su3=su3)
+    for prec, dt, tol in ((Q.F64, np.float64, TOL64), (Q.F32, np.float32, TOL32)):
+        src = p.b.astype(dt)
+        inp = p.lat.spinor(prec, src)
+        want = p.orc.dslash(src, Q.HOPS_ALL, -1, out=np.zeros_like(src))
+        outs = []
+        for k in ((0, 3, 4) if prec == Q.F32 and B == [4, 4, 4, 4] else (None,)):
+            if k is not None:
+                p.lat.set_dslash_kernel(k)
+            out = p.lat.spinor(prec)
+            p.lat.dslash(out, inp, Q.HOPS_ALL, -1)
+            outs.append(out.download())
+        assert rel(outs[0], want) < tol
+        assert all(np.array_equal(outs[0], o) for o in outs)
+        out = p.lat.spinor(prec)
+        for c in (0, 1):
+            p.lat.dslash(out, inp, Q.HOPS_INSIDE, c)
+        for c in (0, 1):
+            p.lat.face(out, inp, -0.125, c)
+        assert rel(out.download(), want) < tol
+
+
+@pytest.mark.parametrize("L,B", [([6, 3, 5, 7], [3, 3, 5, 7]), ([4, 8, 4, 4], [2, 8, 2, 4]),
+                                 ([36, 13, 15, 20], [18, 13, 15, 20])])
+@pytest.mark.parametrize("nsap,nm", [(0, 3), (1, 1), (2, 2)])
+def test_sap_by_steps_with_own_neighbours(L, B, nsap, nm):
+    """SAP on blocks that are their own neighbours in y, z or t, whose unsolved half
+    counts as zero: in one launch per pair of updates, and (2194 groups of 64 sites) in
+    two; out may be the input."""
+    p = Problem(L, B, kappa=0.125, seed=15)
+    bs = p.b.astype(np.float32)
+    x = p.lat.spinor(Q.F32, bs)
+    p.lat.prec_s(x, x, nsap, nm)
+    assert rel(x.download(), p.orc.prec_s(bs, nsap, nm)) < 5e-6
+    x = p.lat.spinor(Q.F32, bs)
+    p.lat.prec_ddd(x, x, nsap, nm)
+    assert rel(x.download(), p.orc.prec_ddd_s(bs, nsap, nm)) < 5e-6
+
+
 @pytest.mark.parametrize("colour", [-1, 0, 1])
 def test_face_accumulate(prob, colour):
     p, lat = prob, prob.lat
