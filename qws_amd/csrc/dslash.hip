@@ -14,6 +14,15 @@ namespace qws {
 
 constexpr int HOP_THREADS = 256;
 
+// Whether the full operator reads its clover and writes its output past the caches (NT).
+// Up to about the last-level cache's 256 MB the operator's data come from there the next
+// time; above, they only push out spinors and links that neighbouring blocks read again
+// (32^3x64 by 4^4 blocks: 1.47 times the bytes needed came from beyond L2).  us with
+// ordinary / nontemporal accesses, 4^4 blocks, FP32 unless said:
+//   198 MB  43.0 / 46.7    226 MB  48.0 / 51.7    264 MB  54.9 / 55.2    297 MB  64.5 / 61.0
+//   340 MB  77.3 / 69.0    446 MB   108 / 88.9   1409 MB   337 / 313     FP64 1019 MB 253 / 235
+constexpr double DSLASH_STREAM_BYTES = 280e6;
+
 template <typename S, int NL, int SET>
 __global__ void __launch_bounds__(HOP_THREADS)
 k_hop(Geo g, const int* __restrict__ list, int wg_per_blk, int nrhs, long long stride, const int* __restrict__ active,
@@ -76,7 +85,7 @@ k_hop(Geo g, const int* __restrict__ list, int wg_per_blk, int nrhs, long long s
 // 3 waves per SIMD (amdgpu_waves_per_eu): the schedule that results orders the
 // neighbour gathers so that FP32 32^3x64 fetches 1.3x less from HBM than the default
 // schedule and runs 2% faster (the register count still admits 5 waves per SIMD).
-template <typename S, int NL>
+template <typename S, int NL, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, 3)))
 k_dslash(Geo g, const int* __restrict__ order, int wg_per_blk, const int* __restrict__ active,
          typename Store<S>::R gamma, S* __restrict__ out, const S* __restrict__ in, const S* __restrict__ U,
@@ -92,12 +101,12 @@ k_dslash(Geo g, const int* __restrict__ order, int wg_per_blk, const int* __rest
   site_coords(g, s, sc);
   Cx<R> acc[12];
   hop_sum<S, NL, HOPS_ALL>(g, s, sc, in, U, acc);
-  clover_apply<S>(C, s, g.V, acc);
+  clover_apply<S, NT>(C, s, g.V, acc);
   Cx<R> v[12];
   SpinorIO<S>::load(in, s, g.V, v);
 #pragma unroll
   for (int k = 0; k < 12; ++k) v[k] = {fmar(gamma, acc[k].re, v[k].re), fmar(gamma, acc[k].im, v[k].im)};
-  SpinorIO<S>::store(out, s, g.V, v);
+  SpinorIO<S>::template store<NT>(out, s, g.V, v);
 }
 
 // One hop of the LDS-staged full operator: the neighbour's spinor from LDS when it
@@ -140,7 +149,7 @@ __device__ __forceinline__ void hop_staged(const Geo& g, long long s, const Site
 // waves per SIMD the compiler schedules for (amdgpu_waves_per_eu); at about 104
 // VGPRs 4 waves are resident either way.
 // (Nontemporal link and clover loads were measured slower here, with more L2 misses.)
-template <int NL, int W>
+template <int NL, int W, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, W)))
 k_dslash_lds(Geo g, const int* __restrict__ order, const int* __restrict__ active, float gamma, float* __restrict__ out,
              const float* __restrict__ in, const float* __restrict__ U, const float* __restrict__ C) {
@@ -165,23 +174,29 @@ k_dslash_lds(Geo g, const int* __restrict__ order, const int* __restrict__ activ
   hop_staged<NL, 2, -1>(g, s, sc, t, lx, in, U, acc);
   hop_staged<NL, 3, +1>(g, s, sc, t, lx, in, U, acc);
   hop_staged<NL, 3, -1>(g, s, sc, t, lx, in, U, acc);
-  clover_apply<float>(C, s, g.V, acc);
-  float4* ov = reinterpret_cast<float4*>(out);
+  clover_apply<float, NT>(C, s, g.V, acc);
+  f4v* ov = reinterpret_cast<f4v*>(out);
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     const float4 o = lx[j * HOP_THREADS + t];
-    ov[(long long)j * g.V + s] = make_float4(fmar(gamma, acc[2 * j].re, o.x), fmar(gamma, acc[2 * j].im, o.y),
-                                             fmar(gamma, acc[2 * j + 1].re, o.z), fmar(gamma, acc[2 * j + 1].im, o.w));
+    st_nt<NT>(ov + ((long long)j * g.V + s), f4v{fmar(gamma, acc[2 * j].re, o.x), fmar(gamma, acc[2 * j].im, o.y),
+                                                 fmar(gamma, acc[2 * j + 1].re, o.z), fmar(gamma, acc[2 * j + 1].im, o.w)});
   }
 }
 
 template <int NL>
 void launch_dslash_lds(const Geo& g, BlockSel sel, const int* active, float gamma, float* out, const float* in,
                        const float* U, const float* C, hipStream_t st) {
-#define DSL_LDS(W) \
-  hipLaunchKernelGGL((k_dslash_lds<NL, W>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, active, gamma, out, in, U, C)
-  if (g.dslash_kernel == 3) DSL_LDS(3);
-  else DSL_LDS(4);
+  const bool nt = operator_bytes<float>(g, NL) > DSLASH_STREAM_BYTES;
+#define DSL_LDS(W, NT) \
+  hipLaunchKernelGGL((k_dslash_lds<NL, W, NT>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, active, gamma, out, in, U, C)
+  if (g.dslash_kernel == 3) {
+    if (nt) DSL_LDS(3, true);
+    else DSL_LDS(3, false);
+  } else {
+    if (nt) DSL_LDS(4, true);
+    else DSL_LDS(4, false);
+  }
 #undef DSL_LDS
 }
 
@@ -217,7 +232,7 @@ __device__ __forceinline__ void hop_staged_d(const Geo& g, long long s, const Si
 
 // FP64 full operator (the outer solver's D, ddd_d_) on 256-site blocks with the block's
 // spinor staged in LDS (12 double2 planes, 48 KB): bit for bit k_dslash<double, 18>.
-template <int W>
+template <int W, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, W)))
 k_dslash_lds_d(Geo g, const int* __restrict__ order, const int* __restrict__ active, double gamma,
                double* __restrict__ out, const double* __restrict__ in, const double* __restrict__ U,
@@ -243,12 +258,12 @@ k_dslash_lds_d(Geo g, const int* __restrict__ order, const int* __restrict__ act
   hop_staged_d<2, -1>(g, s, sc, t, lx, in, U, acc);
   hop_staged_d<3, +1>(g, s, sc, t, lx, in, U, acc);
   hop_staged_d<3, -1>(g, s, sc, t, lx, in, U, acc);
-  clover_apply<double>(C, s, g.V, acc);
-  double2* ov = reinterpret_cast<double2*>(out);
+  clover_apply<double, NT>(C, s, g.V, acc);
+  d2v* ov = reinterpret_cast<d2v*>(out);
 #pragma unroll
   for (int k = 0; k < 12; ++k) {
     const double2 o = lx[k * HOP_THREADS + t];
-    ov[(long long)k * g.V + s] = make_double2(fmar(gamma, acc[k].re, o.x), fmar(gamma, acc[k].im, o.y));
+    st_nt<NT>(ov + ((long long)k * g.V + s), d2v{fmar(gamma, acc[k].re, o.x), fmar(gamma, acc[k].im, o.y)});
   }
 }
 
@@ -263,6 +278,7 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
   }
   if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
     // the full operator: one lean launch per right-hand side
+    const bool nt = operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
     if constexpr (std::is_same<S, float>::value) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel != 0) {
         for (int r = 0; r < B.n; ++r)
@@ -275,20 +291,30 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
       if (g.Vb == HOP_THREADS && g.dslash_kernel_d != 0) {
         for (int r = 0; r < B.n; ++r) {
           const int* act = B.active ? B.active + r : nullptr;
-          if (g.dslash_kernel_d == 2)
-            hipLaunchKernelGGL((k_dslash_lds_d<2>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, act, gamma,
-                               out + r * B.stride, in + r * B.stride, U, C);
-          else
-            hipLaunchKernelGGL((k_dslash_lds_d<3>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, act, gamma,
-                               out + r * B.stride, in + r * B.stride, U, C);
+#define DSL_LDS(W, NT)                                                                                           \
+  hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, act, gamma, \
+                     out + r * B.stride, in + r * B.stride, U, C)
+          if (g.dslash_kernel_d == 2) {
+            if (nt) DSL_LDS(2, true);
+            else DSL_LDS(2, false);
+          } else {
+            if (nt) DSL_LDS(3, true);
+            else DSL_LDS(3, false);
+          }
+#undef DSL_LDS
         }
         return;
       }
     }
     const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
-    for (int r = 0; r < B.n; ++r)
-      hipLaunchKernelGGL((k_dslash<S, NL>), dim3(sel.n * wpb), dim3(HOP_THREADS), 0, st, g, sel.list, wpb,
-                         B.active ? B.active + r : nullptr, gamma, out + r * B.stride, in + r * B.stride, U, C);
+#define DSL(NT)                                                                                         \
+  hipLaunchKernelGGL((k_dslash<S, NL, NT>), dim3(sel.n * wpb), dim3(HOP_THREADS), 0, st, g, sel.list, wpb, \
+                     B.active ? B.active + r : nullptr, gamma, out + r * B.stride, in + r * B.stride, U, C)
+    for (int r = 0; r < B.n; ++r) {
+      if (nt) DSL(true);
+      else DSL(false);
+    }
+#undef DSL
     return;
   }
   const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;

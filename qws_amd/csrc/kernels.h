@@ -8,6 +8,9 @@
 
 namespace qws {
 
+// the fields and spinors of the full operator (4 links, clover, one spinor in and one out)
+template <typename S> double operator_bytes(const Geo& g, int nl) { return (double)g.V * sizeof(S) * (4 * nl + 72 + 48); }
+
 // Blocks to run over: all blocks (list == nullptr) or the blocks of one colour.
 struct BlockSel {
   const int* list;  // device array of block ids, or nullptr for every block

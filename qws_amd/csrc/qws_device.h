@@ -166,6 +166,20 @@ template <> struct Store<float> { using R = float; };
 template <> struct Store<double> { using R = double; };
 template <> struct Store<__half> { using R = float; };
 
+// ---- streams: nontemporal loads and stores of data that one launch reads or writes once,
+// so that the L2 keeps what is read again: the spinors of neighbouring blocks (SAP: links
+// and clover) or sites (the full and the even/odd operators on large lattices).
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef double d2v __attribute__((ext_vector_type(2)));
+template <bool NT = true, typename T> __device__ __forceinline__ T ld_nt(const T* p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
+}
+template <bool NT, typename T> __device__ __forceinline__ void st_nt(T* p, T v) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // ---- spinors
 template <typename S> struct SpinorIO;
 
@@ -179,10 +193,11 @@ template <> struct SpinorIO<float> {
       v[2 * j + 1] = {q.z, q.w};
     }
   }
+  template <bool NT = false>
   static __device__ __forceinline__ void store(float* base, long long s, long long V, const Cx<float> v[12]) {
-    float4* p = reinterpret_cast<float4*>(base);
+    f4v* p = reinterpret_cast<f4v*>(base);
 #pragma unroll
-    for (int j = 0; j < 6; ++j) p[j * V + s] = make_float4(v[2 * j].re, v[2 * j].im, v[2 * j + 1].re, v[2 * j + 1].im);
+    for (int j = 0; j < 6; ++j) st_nt<NT>(p + (j * V + s), f4v{v[2 * j].re, v[2 * j].im, v[2 * j + 1].re, v[2 * j + 1].im});
   }
 };
 
@@ -195,10 +210,11 @@ template <> struct SpinorIO<double> {
       v[k] = {q.x, q.y};
     }
   }
+  template <bool NT = false>
   static __device__ __forceinline__ void store(double* base, long long s, long long V, const Cx<double> v[12]) {
-    double2* p = reinterpret_cast<double2*>(base);
+    d2v* p = reinterpret_cast<d2v*>(base);
 #pragma unroll
-    for (int k = 0; k < 12; ++k) p[k * V + s] = make_double2(v[k].re, v[k].im);
+    for (int k = 0; k < 12; ++k) st_nt<NT>(p + (k * V + s), d2v{v[k].re, v[k].im});
   }
 };
 
@@ -225,21 +241,13 @@ template <> struct SpinorIO<__half> {
       v[2 * j + 1] = {q.z, q.w};
     }
   }
+  template <bool NT = false>
   static __device__ __forceinline__ void store(__half* base, long long s, long long V, const Cx<float> v[12]) {
 #pragma unroll
     for (int j = 0; j < 6; ++j)
       half4_store(base, j * V + s, make_float4(v[2 * j].re, v[2 * j].im, v[2 * j + 1].re, v[2 * j + 1].im));
   }
 };
-
-// ---- streaming loads for the SAP block kernel.  Its links and clover are read once
-// per block and half-sweep and never re-read from L2 within the launch; loading them
-// nontemporally leaves L2 to the spinors of neighbouring blocks.  (The full operator
-// measured slower with them and keeps ordinary loads.)
-typedef float f2v __attribute__((ext_vector_type(2)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ f2v ld_nt(const f2v* p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ f4v ld_nt(const f4v* p) { return __builtin_nontemporal_load(p); }
 
 // ---- links
 template <typename S> __device__ __forceinline__ Cx<typename Store<S>::R> load_cx(const S* base, long long i);
@@ -255,12 +263,16 @@ template <> __device__ __forceinline__ Cx<float> load_cx<__half>(const __half* b
   float2 q = __half22float2(reinterpret_cast<const __half2*>(base)[i]);
   return {q.x, q.y};
 }
-template <typename S> __device__ __forceinline__ Cx<float> load_cx_stream(const S* base, long long i) {
-  return load_cx<S>(base, i);
-}
-template <> __device__ __forceinline__ Cx<float> load_cx_stream<float>(const float* base, long long i) {
-  const f2v q = ld_nt(reinterpret_cast<const f2v*>(base) + i);
-  return {q.x, q.y};
+template <typename S> __device__ __forceinline__ Cx<typename Store<S>::R> load_cx_stream(const S* base, long long i) {
+  if constexpr (std::is_same<S, float>::value) {
+    const f2v q = ld_nt(reinterpret_cast<const f2v*>(base) + i);
+    return {q.x, q.y};
+  } else if constexpr (std::is_same<S, double>::value) {
+    const d2v q = ld_nt(reinterpret_cast<const d2v*>(base) + i);
+    return {q.x, q.y};
+  } else {
+    return load_cx<S>(base, i);
+  }
 }
 
 // row 2 of a 12-real link = conj(row0 x row1) (wilson_d.h:160-171)
@@ -271,12 +283,12 @@ template <typename R> __device__ __forceinline__ void link_row2(Cx<R> u[9]) {
 }
 
 // u[i*3+j] = QWS c[i][j] of the link at site s, direction mu.
-template <typename S, int NL>
+template <typename S, int NL, bool STREAM = false>
 __device__ __forceinline__ void load_link(const S* U, int mu, long long s, long long V, Cx<typename Store<S>::R> u[9]) {
   constexpr int NC = NL / 2;
   const long long base = (long long)mu * NC * V + s;
 #pragma unroll
-  for (int k = 0; k < NC; ++k) u[k] = load_cx<S>(U, base + k * V);
+  for (int k = 0; k < NC; ++k) u[k] = STREAM ? load_cx_stream<S>(U, base + k * V) : load_cx<S>(U, base + k * V);
   if (NL == 12) link_row2(u);
 }
 
@@ -360,22 +372,24 @@ template <> struct CloverIO<float> {
 #pragma unroll
     for (int f = 0; f < 9; ++f) {
       const f4v* q = p + (long long)(9 * i + f) * V + s;
-      const f4v v = STREAM ? ld_nt(q) : *q;
+      const f4v v = ld_nt<STREAM>(q);
       a[4 * f] = v.x; a[4 * f + 1] = v.y; a[4 * f + 2] = v.z; a[4 * f + 3] = v.w;
     }
   }
 };
 template <> struct CloverIO<double> {
+  template <bool STREAM = false>
   static __device__ __forceinline__ void load_chir(const double* C, long long s, long long V, int i, double a[36]) {
-    const double2* p = reinterpret_cast<const double2*>(C);
+    const d2v* p = reinterpret_cast<const d2v*>(C);
 #pragma unroll
     for (int f = 0; f < 18; ++f) {
-      double2 q = p[(long long)(18 * i + f) * V + s];
+      const d2v q = ld_nt<STREAM>(p + ((long long)(18 * i + f) * V + s));
       a[2 * f] = q.x; a[2 * f + 1] = q.y;
     }
   }
 };
 template <> struct CloverIO<__half> {
+  template <bool STREAM = false>
   static __device__ __forceinline__ void load_chir(const __half* C, long long s, long long V, int i, float a[36]) {
 #pragma unroll
     for (int f = 0; f < 9; ++f) {
@@ -403,7 +417,7 @@ __device__ __forceinline__ void herm6_mult(const R a[36], const Cx<R> x[6], Cx<R
     }
 }
 
-template <typename S>
+template <typename S, bool STREAM = false>
 __device__ __forceinline__ void clover_apply(const S* C, long long s, long long V, Cx<typename Store<S>::R> v[12]) {
   using R = typename Store<S>::R;
   Cx<R> x[6], y0[6], y1[6];
@@ -411,11 +425,11 @@ __device__ __forceinline__ void clover_apply(const S* C, long long s, long long 
   // chirality 0: x = (s0+s2, s1+s3)
 #pragma unroll
   for (int c = 0; c < 3; ++c) { x[c] = cadd(v[c * 4 + 0], v[c * 4 + 2]); x[3 + c] = cadd(v[c * 4 + 1], v[c * 4 + 3]); }
-  CloverIO<S>::load_chir(C, s, V, 0, a);
+  CloverIO<S>::template load_chir<STREAM>(C, s, V, 0, a);
   herm6_mult(a, x, y0);
 #pragma unroll
   for (int c = 0; c < 3; ++c) { x[c] = csub(v[c * 4 + 0], v[c * 4 + 2]); x[3 + c] = csub(v[c * 4 + 1], v[c * 4 + 3]); }
-  CloverIO<S>::load_chir(C, s, V, 1, a);
+  CloverIO<S>::template load_chir<STREAM>(C, s, V, 1, a);
   herm6_mult(a, x, y1);
 #pragma unroll
   for (int c = 0; c < 3; ++c) {

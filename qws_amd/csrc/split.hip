@@ -290,7 +290,7 @@ k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2
 //                    24^3 32, 4^4 blocks (6912) 78.3 / 80.0    163 / 163: to 4096
 //                    16^3 8, 4^4 blocks (512)   14.5 / 7.7      19.1 / 13.0
 //                    32 12^2 10, halves (720)  11.8 / 10.0      17.0 / 19.3
-//                    48 24^3, halves (10368)  134.7 / 125.6      306 / 256
+//                    48 24^3, halves (10368)   93.2 / 107        285 / 255: FP32 to 4096
 //   inside           48 24^3, halves (5184)    59.4 / 50.6       129 / 117
 //   (32^3 64 by halves is the same either way, by 4^4 blocks up to 8% slower here)
 //   faces            16^4, 4^4 blocks (512)    12.7 / 7.5       16.7 / 12.7
@@ -307,7 +307,7 @@ bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64) {
   if (set == HOPS_FACE || g.Vb < SITES) return wg <= 1024;
   if (fp64 && set == HOPS_ALL && wg > 512 && wg < 1024) return false;
   if (nrhs > 1) return wg <= 2048;
-  return wg <= (set == HOPS_ALL && g.Vb == 256 ? 4096 : 16384);
+  return wg <= (set == HOPS_ALL && (g.Vb == 256 || !fp64) ? 4096 : 16384);
 }
 
 template <typename S, int NL>
