@@ -16,7 +16,7 @@
 // Bound by the latency of a Jacobi step: two waves per SIMD, four barriers, 975 vector
 // instructions per wave in 7400 cycles, as long with one workgroup on the CU as with two.
 // More waves do not fit: links, clover, source and sum take 251 of 256 registers.
-// A launch on 2048 blocks (half of 32^3 x 64; nm 6), general kernel / this one: 12-real links
+// A launch on 4096 blocks (half of 32^3 x 64; nm 6), general kernel / this one: 12-real links
 // 0.335 / 0.306 ms, 18-real (which the general kernel reads from memory at each hop)
 // 0.564 / 0.314 ms; on 8 blocks (8^4) 0.0316 / 0.0285 ms.
 #include <type_traits>
@@ -287,7 +287,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
   // The two workgroups of a CU would load, solve and write at the same time: in a launch
   // of several rounds the second ones start half a block's time late (a sleep of about
   // 1 us each turn), so that one computes while the other waits for memory.  SAP launch,
-  // without and with it (nm 6): 2048 blocks 0.316 / 0.308 ms, 1024 blocks 0.170 / 0.162;
+  // without and with it (nm 6): 4096 blocks 0.316 / 0.308 ms, 2048 blocks 0.170 / 0.162;
   // 512 blocks, a single round, 0.049 / 0.055, so not there.
   if (gridDim.x >= 1024 && blockIdx.x >= 256 && blockIdx.x < 512)
     for (int i = 6 + nm * 8 / 5; i > 0; --i) __builtin_amdgcn_s_sleep(37);
@@ -432,7 +432,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
           o = xk - kappa * ak;
           if (epi == SAP_EPI_OUT_FACE) o = o + (iv[k] - sk);
         }
-        (po + k * g.V)[te] = o;
+        st_nt<true>((po + k * g.V) + te, o);
         fence();
       }
     } else {
