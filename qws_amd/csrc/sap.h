@@ -60,7 +60,7 @@ template <typename S> struct SapMulti {
 };
 
 bool sap_fusable(const Geo& g);
-// 4^4 blocks: the FP32 kernel of sap4.hip
+// 4^4 blocks: the kernels of sap4.hip and sap4h.hip
 bool sap_is_4444(const Geo& g);
 // floats per RHS of the face buffer, or 0 when the block shape does not allow it
 // (its slots must fit the iterate's LDS: 2 sum_mu Vb / B_mu <= 2 Vb)
@@ -81,6 +81,10 @@ void launch_sap_4444(const Geo& g, BlockSel sel, const Batch& B, int nl, float k
                      const float* in, const float* qface, float* qout, float* out, const float* U, const float* C,
                      float* fb, long long fbs, hipStream_t st, const SapSrcUpdate& upd);
 void launch_sap_4444_multi(const SapMulti<float>& m, int nl, int nm, int flags, hipStream_t st);
+// launch_sap_block<__half> on 4^4 blocks (sap4h.hip)
+void launch_sap_4444_h(const Geo& g, BlockSel sel, const Batch& B, int nl, float kappa, int nm, int flags, __half* s,
+                       const __half* in, const __half* qface, __half* qout, __half* out, const __half* U, const __half* C,
+                       float* fb, long long fbs, hipStream_t st);
 // launch_sap_face over several lattices (part.out, .fb, .fbs, .U, .C; factor in .kappa)
 void launch_sap_face_multi(const SapMulti<float>& m, int vb, int nl, hipStream_t st);
 

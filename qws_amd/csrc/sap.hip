@@ -59,12 +59,13 @@ void launch_sap_block(const Geo& g, BlockSel sel, const Batch& B, int nl, float 
         (const void*)upd.p != (const void*)in)
       throw std::invalid_argument("fused SAP: the source update needs FP32, SAP_SRC_IN and in == p, r, q, scalars");
   }
-  if constexpr (std::is_same<S, float>::value) {
-    if (sap_is_4444(g)) {
-      check_face_flags(flags);
+  if (sap_is_4444(g)) {
+    check_face_flags(flags);
+    if constexpr (std::is_same<S, float>::value)
       launch_sap_4444(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);
-      return;
-    }
+    else
+      launch_sap_4444_h(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st);
+    return;
   }
   if (g.Vb == 512) sap512::launch<S>(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);
   else sap256::launch<S>(g, sel, B, nl, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, st, upd);

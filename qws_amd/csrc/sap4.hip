@@ -23,38 +23,13 @@
 
 #include "kernels.h"
 #include "sap.h"
-#include "sap_device.h"
+#include "sap4_device.h"
 
 namespace qws {
 
+using namespace sap4;
+
 namespace {
-
-constexpr int VB = 256;  // sites per block = threads per workgroup
-constexpr int FS = 512;  // face slots per block (sap_kernels.inc has their order)
-
-// Position of block site s = (x, y, z, t) in an LDS plane of float4: its low four bits
-// (x, y) XORed by a constant for each z.  A 128-bit LDS read serves lanes 0-3, 12-15 and
-// 20-27 (then the others of 32) at once from 16 groups of 16 bytes, a write eight lanes in
-// a row from 8 groups; with these constants, and the lane order of link_site, every access
-// of block_hops is free of bank conflicts.
-__device__ __forceinline__ int lds_pos(int s) { return s ^ ((0x7AD0 >> ((s >> 2) & 12)) & 15); }
-
-// The site with coordinate l along mu whose other coordinates are those of lane j, the
-// first of them fastest (the order of the face slots).
-__device__ __forceinline__ int slice_site(int mu, int l, int j) {
-  if (mu == 0) return l + 4 * j;
-  if (mu == 1) return (j & 3) + 4 * l + 16 * (j >> 2);
-  if (mu == 2) return (j & 15) + 16 * l + 64 * (j >> 4);
-  return j + 64 * l;
-}
-// The same for the links inside the block; along x the lane bits are y0 z0 z1 y1 t0 t1.
-__device__ __forceinline__ int link_site(int mu, int l, int j) {
-  return slice_site(mu, l, mu == 0 ? (j & 0x31) | ((j & 6) << 1) | ((j & 8) >> 2) : j);
-}
-
-// Nothing is scheduled across this: keeps LDS reads where they are issued, ahead of the
-// arithmetic that hides their latency.
-__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 
 // What the hop along MU, DIR takes of the spinor at LDS position p: all six planes, or
 // for t the spins 2, 3 (forward: planes 1, 3, 5) or 0, 1 (0, 2, 4).
@@ -77,33 +52,6 @@ __device__ __forceinline__ void project_raw(const Raw& r, Cx<float> a[6]) {
     v[2 * k + 1] = on ? Cx<float>{r.q[k].z, r.q[k].w} : Cx<float>{0, 0};
   }
   project<float, MU, DIR>(v, a);
-}
-
-__device__ __forceinline__ void store_half(f4v* lh, int mu, int p, const Cx<float> h[6]) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    lh[(mu * 3 + k) * VB + p] = f4v{h[2 * k].re, h[2 * k].im, h[2 * k + 1].re, h[2 * k + 1].im};
-}
-
-// The half spinors of the four directions at position p, and their sums into the site.
-struct Halves {
-  f4v q[4][3];
-};
-__device__ __forceinline__ void read_halves(const f4v* lh, int p, Halves& h) {
-#pragma unroll
-  for (int mu = 0; mu < 4; ++mu)
-#pragma unroll
-    for (int k = 0; k < 3; ++k) h.q[mu][k] = lh[(mu * 3 + k) * VB + p];
-}
-template <int MU, int DIR>
-__device__ __forceinline__ void add_half(const Halves& hs, float tf, Cx<float> acc[12]) {
-  Cx<float> h[6];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    h[2 * k] = {hs.q[MU][k].x, hs.q[MU][k].y};
-    h[2 * k + 1] = {hs.q[MU][k].z, hs.q[MU][k].w};
-  }
-  reconstruct<float, MU, DIR>(h, tf, acc);
 }
 
 // A wave's links and where their ends lie in the LDS planes.
@@ -138,20 +86,6 @@ __device__ __forceinline__ void tasks(const f4v* lx, f4v* lh, const WaveLinks& w
   project_raw<M2, DIR>(r, a);
   link_mult<float, DIR>(w.u[2], a, h);
   store_half(lh, M2, to<DIR>(w, 2), h);
-}
-
-// The thread's index, as a value that the compiler computes anew where it is asked for:
-// what derives from it (addresses, coordinates) is not kept in registers meanwhile.
-__device__ __forceinline__ unsigned fresh_thread() {
-  unsigned t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
-struct Coord {
-  int x, y, z, t;
-};
-__device__ __forceinline__ Coord coord(unsigned t, int wave) {
-  return {(int)(t & 3), (int)((t >> 2) & 3), (int)((t >> 4) & 3), wave};
 }
 
 // acc = H_in x for the iterate in lx at this thread's site (position p).
@@ -212,29 +146,6 @@ __device__ __forceinline__ void load_site(const float* f, long long first, long 
     v[2 * k] = {q.x, q.y};
     v[2 * k + 1] = {q.z, q.w};
   }
-}
-
-// A wave's slots of the face update, direction MU = its own number: the + side's half
-// spinors in q[0..2], the - side's in q[3..5].
-__device__ __forceinline__ void read_slots(const f4v* slots, int wave, unsigned j, f4v q[6]) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    q[k] = (slots + k * FS + wave * 128)[j];
-    q[3 + k] = (slots + k * FS + wave * 128 + 64)[j];
-  }
-}
-// Its share of the face update: the + side through this face's links (the hop lands on
-// l = 3, position p3), the - side as it is (l = 0).
-__device__ __forceinline__ void face_stage(const f4v q[6], int wave, f4v* lh, int p3, int p0, const Cx<float> u[9]) {
-  Cx<float> a[6], h[6];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    lh[(wave * 3 + k) * VB + p0] = q[3 + k];
-    a[2 * k] = {q[k].x, q[k].y};
-    a[2 * k + 1] = {q[k].z, q[k].w};
-  }
-  link_mult<float, +1>(u, a, h);
-  store_half(lh, wave, p3, h);
 }
 
 // Wave MU's share of the face buffer for the next launch: this block's l = 0 sites as

@@ -58,6 +58,26 @@ def test_msap_h_matches_oracle(prob, nsap, nm):
         assert rel(got, p.orc.prec_s(b, nsap, nm)) > 5 * TOL_H
 
 
+@pytest.mark.parametrize("su3", [True, False])
+@pytest.mark.parametrize("L,nsap,nm", [([8, 8, 8, 8], 2, 1), ([24, 8, 16, 8], 4, 2), ([24, 8, 16, 8], 1, 5)])
+def test_msap_h_4444(L, nsap, nm, su3):
+    """The FP16 kernel for 4^4 blocks (hops by link) where both neighbours of a block are
+    the same one, at extents that differ in every direction, with one Jacobi step and
+    several: the oracle's result, by the face buffer bit for bit as by gathers, to the
+    FP16 tolerance of the tests here."""
+    p = Problem(L, [4, 4, 4, 4], su3=su3)
+    b = p.b.astype(np.float32)
+    res = []
+    for fb in (True, False):
+        p.lat.set_sap_face_buffer(fb)
+        out = p.lat.spinor(Q.F32)
+        p.lat.msap_h(out, p.lat.spinor(Q.F32, b), nsap, nm)
+        res.append(out.download())
+    p.lat.set_sap_face_buffer(True)
+    assert np.array_equal(*res)
+    assert rel(res[0], p.orc.msap_h(b, nsap, nm)) < 2 * TOL_H
+
+
 @pytest.mark.parametrize("L,B,su3", [([16, 8, 8, 8], [4, 4, 4, 4], True), ([16, 8, 8, 8], [4, 4, 4, 4], False),
                                      ([16, 8, 8, 8], [8, 4, 4, 4], True)])
 def test_msap_h_face_buffer_is_bitwise_the_gather(L, B, su3):
