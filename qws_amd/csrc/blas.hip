@@ -236,14 +236,14 @@ __device__ __forceinline__ void cdiv(double ar, double ai, double br, double bi,
 // Deterministic sum of the partials of RHS blockIdx.x, then the scalar
 // recurrences of BiCGStab with the reference's breakdown guards
 // (bicgstab_dd_mix.cc:192,279,359).
-__global__ void __launch_bounds__(RED_THREADS) k_finalize(const double* part, int nval, Scalars* scs, int mode,
-                                                          const int* active) {
+__global__ void __launch_bounds__(RED_THREADS) k_finalize(const double* part, int count, int nval, Scalars* scs,
+                                                          int mode, const int* active) {
   const int r = blockIdx.x;
   if (active && !active[r]) return;
   __shared__ double sh[4][RED_THREADS];
   for (int v = 0; v < nval; ++v) {
     double x = 0;
-    for (int i = threadIdx.x; i < RED_BLOCKS; i += RED_THREADS) x += part[((long long)r * 4 + v) * RED_BLOCKS + i];
+    for (int i = threadIdx.x; i < count; i += RED_THREADS) x += part[((long long)r * 4 + v) * count + i];
     sh[v][threadIdx.x] = x;
   }
   __syncthreads();
@@ -469,8 +469,8 @@ template <typename R>
 void launch_norm(const Batch& B, long long n, const R* a, double* part, hipStream_t st) {
   LAUNCH_B((k_norm<R>), B.n, n, B.stride, B.active, a, part);
 }
-void launch_finalize(const Batch& B, const double* part, int nval, Scalars* sc, int mode, hipStream_t st) {
-  hipLaunchKernelGGL(k_finalize, dim3(B.n), dim3(RED_THREADS), 0, st, part, nval, sc, mode, B.active);
+void launch_finalize(const Batch& B, const double* part, int nval, Scalars* sc, int mode, hipStream_t st, int count) {
+  hipLaunchKernelGGL(k_finalize, dim3(B.n), dim3(RED_THREADS), 0, st, part, count, nval, sc, mode, B.active);
 }
 template <typename S>
 void launch_d2s_scaled(const Batch& B, long long V, long long so, long long si, S* out, const double* in,

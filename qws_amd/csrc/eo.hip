@@ -11,9 +11,11 @@
 //   links   [2][4][NL/2][Vh] Vec2  (link from site h of parity p)
 //   clover  [2][18][Vh] float4 / [2][36][Vh] double2
 // One thread per site of the output parity.
+#include <stdexcept>
 #include <type_traits>
 
 #include "kernels.h"
+#include "split_device.h"
 
 namespace qws {
 
@@ -76,19 +78,51 @@ __device__ __forceinline__ void eo_hop(const Geo& g, int pe, long long h, const 
   reconstruct<R, MU, PD>(b, tf, acc);
 }
 
+// Reductions of out that BiCGStab takes next, in FP64 without another pass over it:
+// <z, out> (DEO_DOT) or |out|^2 and <out, in0> (DEO_NORM_DOT).
+template <int RED, typename R>
+__device__ __forceinline__ void deo_reduce(Cx<R> o, Cx<R> w, double acc[3]) {
+  if (RED == DEO_DOT) {
+    acc[0] += (double)w.re * o.re + (double)w.im * o.im;
+    acc[1] += (double)w.re * o.im - (double)w.im * o.re;
+  } else if (RED == DEO_NORM_DOT) {
+    acc[0] += (double)o.re * o.re + (double)o.im * o.im;
+    acc[1] += (double)o.re * w.re + (double)o.im * w.im;
+    acc[2] += (double)o.re * w.im - (double)o.im * w.re;
+  }
+}
+// the workgroup's sums: part[v * gridDim.x + blockIdx.x]
+template <int RED> __device__ __forceinline__ void deo_partials(const double acc[3], double* part) {
+  __shared__ double sh[3][EO_THREADS / 64];
+  constexpr int NV = RED == DEO_DOT ? 2 : 3;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    double x = acc[v];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[v][threadIdx.x >> 6] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV)
+    part[(long long)threadIdx.x * gridDim.x + blockIdx.x] =
+        ((sh[threadIdx.x][0] + sh[threadIdx.x][1]) + sh[threadIdx.x][2]) + sh[threadIdx.x][3];
+}
+
 // For every site h of parity pe: acc = sum of the hops of `set` (0 all, 1 no wrap,
 // 2 wrap only, 3 none: acc = in[h]) from in; clv: acc = T^-1 acc; then
 // mode 0: out = acc, 1: out += fac acc, 2: out = in0 + fac acc.
-template <typename S, int NL, bool DAG, bool NT>
+template <typename S, int NL, bool DAG, bool NT, int RED>
 __global__ void __launch_bounds__(EO_THREADS)
 k_deo(Geo g, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out, const S* __restrict__ in,
-      const S* in0, const S* __restrict__ U, const S* __restrict__ C) {
+      const S* in0, const S* __restrict__ U, const S* __restrict__ C, const S* z, double* part) {
   using R = typename Store<S>::R;
   const long long Vh = g.V >> 1;
   // XCD-contiguous ranges of sites: the z and t neighbours a workgroup reads were fetched
   // by workgroups on the same XCD (its L2), not by ones spread round-robin over the XCDs
-  const long long h = xcd_remap(g, blockIdx.x, gridDim.x) * (long long)EO_THREADS + threadIdx.x;
-  if (h >= Vh) return;
+  long long h = xcd_remap(g, blockIdx.x, gridDim.x) * (long long)EO_THREADS + threadIdx.x;
+  const bool on = h < Vh;
+  if (RED == DEO_STORE && !on) return;
+  if (!on) h = Vh - 1;  // (idle, but there for the sums)
   EoSite e;
   eo_coords(g, pe, h, e);
   Cx<R> acc[12];
@@ -107,28 +141,210 @@ k_deo(Geo g, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* ou
     eo_hop<S, NL, 3, -1, DAG, NT>(g, pe, h, e, set, in, U, Vh, acc);
   }
   if (clv) clover_apply<S, NT>(C + (long long)pe * 72 * Vh, h, Vh, acc);
+  double red[3] = {0, 0, 0};
   if (mode != 0) {
     Cx<R> o[12];
     SpinorIO<S>::load(mode == 1 ? out : in0, h, Vh, o);
 #pragma unroll
     for (int k = 0; k < 12; ++k) acc[k] = cadd(o[k], cscale(fac, acc[k]));
+    if (RED == DEO_DOT) SpinorIO<S>::load(z, h, Vh, o);
+    if (RED != DEO_STORE && on) {
+#pragma unroll
+      for (int k = 0; k < 12; ++k) deo_reduce<RED>(acc[k], o[k], red);
+    }
   }
-  SpinorIO<S>::template store<NT>(out, h, Vh, acc);
+  if (RED == DEO_STORE || on) SpinorIO<S>::template store<NT>(out, h, Vh, acc);
+  if (RED != DEO_STORE) deo_partials<RED>(red, part);
 }
 
-template <typename S>
-void launch_deo(const Geo& g, int nl, int pe, int set, int dag, int clv, int mode, typename Store<S>::R fac, S* out,
-                const S* in, const S* in0, const S* U, const S* C, hipStream_t st) {
+// k_deo (sets 0 to 2) with four waves per 64 sites, for few sites: as k_split of split.hip.
+template <typename S, int NL, int MU, bool DAG, typename Rest>
+__device__ __forceinline__ void eo_two_hops(const Geo& g, int pe, int h, int first, const EoSite& e, bool on, int set,
+                                            const S* in, const S* U, Cx<typename Store<S>::R> (*lh)[6][split::SITES],
+                                            Rest&& rest) {
+  using R = typename Store<S>::R;
+  using IO = split::IO<S>;
+  constexpr int NC = NL / 2, BOTH = sizeof(S) == 8 ? 0 : 1;
+  const int lane = threadIdx.x & 63, Vh = (int)(g.V >> 1), nxh = g.L[0] >> 1;
+  const int step = MU == 0 ? 1 : MU == 1 ? nxh : MU == 2 ? nxh * g.L[1] : nxh * g.L[1] * g.L[2];
+  Cx<R> v[1 + BOTH][12], u[1 + BOTH][9];
+  bool take[2];
+  auto load = [&](int d) {
+    const int ext = MU == 0 ? nxh : g.L[MU], dir = d == 0 ? 1 : -1;
+    const int c = e.c[MU] + (MU == 0 ? (d == 0 ? e.ick : e.ick - 1) : dir);
+    const bool wraps = c < 0 || c >= ext;
+    const int n = h + ((c < 0 ? ext - 1 : c >= ext ? 0 : c) - e.c[MU]) * step;
+    take[d] = on && !((set == 1 && wraps) || (set == 2 && !wraps));
+    if (!__any(take[d])) return;
+    const unsigned nn = take[d] ? n : first, at = d == 0 ? (take[d] ? h : first) : nn;
+    const S* Ub = U + (long long)(d == 0 ? pe : 1 - pe) * 4 * NL * Vh;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) IO::load2(in, j, Vh, nn * IO::Q, v[d * BOTH] + 2 * j);
+#pragma unroll
+    for (int k = 0; k < NC; ++k) u[d * BOTH][k] = IO::link(Ub, MU * NC + k, Vh, at * split::LINK_BYTES<S>);
+  };
+  auto hop = [&](int d) {
+    Cx<R> o[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[k] = {0, 0};
+    if (__any(take[d])) {
+      Cx<R> a[6], m[6];
+      if (NL == 12) link_row2(u[d * BOTH]);
+      if (d == 0) {
+        project<R, MU, DAG ? -1 : +1>(v[d * BOTH], a);
+        link_mult<R, +1>(u[d * BOTH], a, m);
+      } else {
+        project<R, MU, DAG ? +1 : -1>(v[d * BOTH], a);
+        link_mult<R, -1>(u[d * BOTH], a, m);
+      }
+#pragma unroll
+      for (int k = 0; k < 6; ++k) o[k] = {take[d] ? m[k].re : R(0), take[d] ? m[k].im : R(0)};
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) lh[2 * MU + d][k][lane] = o[k];
+  };
+  asm volatile("; hops of direction %0" ::"i"(MU));  // (the four waves' branches are not merged)
+  load(0);
+  if (BOTH) load(1);
+  if (BOTH) rest();
+  __builtin_amdgcn_sched_barrier(0);
+  hop(0);
+  if (!BOTH) {
+    load(1);
+    hop(1);
+    rest();
+  } else {
+    hop(1);
+  }
+  asm volatile("; end of direction %0" ::"i"(MU));
+}
+
+template <typename S, int NL, bool DAG, int RED>
+__global__ void __launch_bounds__(256, 2)
+k_deo_split(Geo g, float rnx, float ry, float rz, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out,
+            const S* __restrict__ in, const S* in0, const S* __restrict__ U, const S* __restrict__ C, const S* z,
+            double* part) {
+  using R = typename Store<S>::R;
+  using IO = split::IO<S>;
+  constexpr int SITES = split::SITES;
+  __shared__ Cx<R> lh[8][6][SITES];
+  __shared__ Cx<R> ly[12][SITES];
+  const int lane = threadIdx.x & 63, Vh = (int)(g.V >> 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int first = xcd_remap(g, blockIdx.x, gridDim.x) * SITES;
+  const bool on = first + lane < Vh;
+  const int h = on ? first + lane : first;
+  EoSite e;
+  {
+    // quotients by the reciprocal: exact below 2^20
+    const int nxh = g.L[0] >> 1;
+    const int q0 = (int)((h + 0.5f) * rnx), q1 = (int)((q0 + 0.5f) * ry), q2 = (int)((q1 + 0.5f) * rz);
+    e.c[0] = h - q0 * nxh, e.c[1] = q0 - q1 * g.L[1], e.c[2] = q1 - q2 * g.L[2], e.c[3] = q2;
+    e.ick = (pe + e.c[1] + e.c[2] + e.c[3]) & 1;
+  }
+  const unsigned at = (unsigned)h * IO::Q;
+  R ca[36];  // chirality wave & 1 of T^-1
+  auto rest = [&]() { IO::chir(C + (long long)pe * 72 * Vh, wave & 1, Vh, at, ca); };  // (unused without clv)
+  if (wave == 0) eo_two_hops<S, NL, 0, DAG>(g, pe, h, first, e, on, set, in, U, lh, rest);
+  else if (wave == 1) eo_two_hops<S, NL, 1, DAG>(g, pe, h, first, e, on, set, in, U, lh, rest);
+  else if (wave == 2) eo_two_hops<S, NL, 2, DAG>(g, pe, h, first, e, on, set, in, U, lh, rest);
+  else eo_two_hops<S, NL, 3, DAG>(g, pe, h, first, e, on, set, in, U, lh, rest);
+  __syncthreads();
+  Cx<R> acc[12], b[6];
+#pragma unroll
+  for (int k = 0; k < 12; ++k) acc[k] = {0, 0};
+  const R tf_hi = e.c[3] == g.L[3] - 1 ? (R)(2 * g.tbc) : R(2), tf_lo = e.c[3] == 0 ? (R)(2 * g.tbc) : R(2);
+#define ADD(MU, DIR, TF)                                                                       \
+  _Pragma("unroll") for (int k = 0; k < 6; ++k) b[k] = lh[2 * MU + (DIR < 0)][k][lane];        \
+  reconstruct<R, MU, DAG ? -(DIR) : DIR>(b, TF, acc);
+  ADD(0, +1, R(2)) ADD(0, -1, R(2)) ADD(1, +1, R(2)) ADD(1, -1, R(2))
+  ADD(2, +1, R(2)) ADD(2, -1, R(2)) ADD(3, +1, tf_hi) ADD(3, -1, tf_lo)
+#undef ADD
+  // wave c < 3 stores colour c; its term of the output, and of the sums
+  Cx<R> o[2][2], w[2][2];
+  auto terms = [&]() {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (mode != 0) IO::load2(mode == 1 ? out : in0, 2 * wave + j, Vh, at, o[j]);
+      if (RED == DEO_DOT) IO::load2(z, 2 * wave + j, Vh, at, w[j]);
+    }
+  };
+  if (sizeof(S) == 4 && wave < 3) terms();  // (FP64 has no registers for them yet)
+  if (clv) {
+    Cx<R> x[6], y[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      if (wave & 1) x[c] = csub(acc[c * 4], acc[c * 4 + 2]), x[3 + c] = csub(acc[c * 4 + 1], acc[c * 4 + 3]);
+      else x[c] = cadd(acc[c * 4], acc[c * 4 + 2]), x[3 + c] = cadd(acc[c * 4 + 1], acc[c * 4 + 3]);
+    }
+    if (wave < 2) split::herm3_mult<0>(ca, x, y);
+    else split::herm3_mult<1>(ca, x, y);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) ly[(wave & 1) * 6 + (wave >> 1) * 3 + k][lane] = y[k];
+  } else if (wave == 0) {  // as the two chiralities whose combination is acc
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      ly[c][lane] = acc[4 * c], ly[3 + c][lane] = acc[4 * c + 1];
+      ly[6 + c][lane] = acc[4 * c + 2], ly[9 + c][lane] = acc[4 * c + 3];
+    }
+  }
+  __syncthreads();
+  double red[3] = {0, 0, 0};
+  if (wave < 3 && on) {
+    if (sizeof(S) == 8) terms();
+    const Cx<R> y0 = ly[wave][lane], y1 = ly[3 + wave][lane], z0 = ly[6 + wave][lane], z1 = ly[9 + wave][lane];
+    Cx<R> t[2][2] = {{y0, y1}, {z0, z1}};
+    if (clv) t[0][0] = cadd(y0, z0), t[0][1] = cadd(y1, z1), t[1][0] = csub(y0, z0), t[1][1] = csub(y1, z1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (mode != 0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          t[j][k] = cadd(o[j][k], cscale(fac, t[j][k]));
+          if (RED != DEO_STORE) deo_reduce<RED>(t[j][k], RED == DEO_DOT ? w[j][k] : o[j][k], red);
+        }
+      }
+      IO::store2(out, 2 * wave + j, Vh, at, t[j]);
+    }
+  }
+  if (RED != DEO_STORE) deo_partials<RED>(red, part);
+}
+
+// Whether k_deo_split is the faster one: by its workgroups (64 sites).  mtilde in us with
+// k_deo / with it, 18-real links:
+//   workgroups   32          256         512         768         1024        1536        2048        3456
+//   FP32         16.8 / 9.8  17.4 / 10.5 23.4 / 14.7 25.8 / 20.4 28.4 / 26.5 35.2 / 36.0 44.0 / 46.8 94.4 / 76.1
+//   FP64         19.8 / 11.3 25.7 / 14.9 30.4 / 27.1 36.2 / 37.9 52.2 / 50.1 84 / 70     100 / 100   181 / 201
+// FP32 also wins from three full rounds on (768 workgroups each; 2304: 53.6 / 50.7) to 4096
+// (5184: 145 / 151); FP64's gains past 512 come and go with its rounds of 512.
+static int deo_split_groups(const Geo& g) { return (int)(((g.V >> 1) + split::SITES - 1) / split::SITES); }
+static bool deo_split_pays(const Geo& g, int set, bool fp64) {
+  const int n = deo_split_groups(g);
+  if (set == 3 || (g.V >> 1) >= (1 << 20)) return false;
+  return fp64 ? n <= 512 : n <= 1280 || (n >= 2304 && n <= 4096);
+}
+
+template <typename S, int RED>
+static void deo_launch(const Geo& g, int nl, int pe, int set, int dag, int clv, int mode, typename Store<S>::R fac, S* out,
+                       const S* in, const S* in0, const S* U, const S* C, const S* z, double* part, hipStream_t st) {
   const long long Vh = g.V >> 1;
   dim3 grid((unsigned)((Vh + EO_THREADS - 1) / EO_THREADS)), block(EO_THREADS);
-#define DEO_ARGS g, pe, set, clv, mode, fac, out, in, in0, U, C
+  const bool sp = deo_split_pays(g, set, sizeof(S) == 8);
+  if (sp) grid = dim3(deo_split_groups(g));
   const bool nt = (double)g.V * sizeof(S) * (4 * nl + 36 + 24) > DEO_STREAM_BYTES;
-#define DEO(NL, DAG)                                                                            \
-  do {                                                                                         \
-    if (nt) hipLaunchKernelGGL((k_deo<S, NL, DAG, true>), grid, block, 0, st, DEO_ARGS); \
-    else hipLaunchKernelGGL((k_deo<S, NL, DAG, false>), grid, block, 0, st, DEO_ARGS);         \
+#define DEO_ARGS pe, set, clv, mode, fac, out, in, in0, U, C, z, part
+#define DEO(NL, DAG)                                                                                                 \
+  do {                                                                                                               \
+    if (sp)                                                                                                          \
+      hipLaunchKernelGGL((k_deo_split<S, NL, DAG, RED>), grid, block, 0, st, g, 2.0f / g.L[0], 1.0f / g.L[1],        \
+                         1.0f / g.L[2], DEO_ARGS);                                                                   \
+    else if (nt) hipLaunchKernelGGL((k_deo<S, NL, DAG, true, RED>), grid, block, 0, st, g, DEO_ARGS);                \
+    else hipLaunchKernelGGL((k_deo<S, NL, DAG, false, RED>), grid, block, 0, st, g, DEO_ARGS);                       \
   } while (0)
-  if (sizeof(S) == 4 && nl == 12) {
+  if constexpr (RED != DEO_STORE) {
+    if (nl != 18 || dag || set != 0 || mode != 2) throw std::logic_error("deo_launch: sums with the FP64 operator only");
+    DEO(18, false);
+  } else if (sizeof(S) == 4 && nl == 12) {
     if constexpr (std::is_same<S, float>::value) {
       if (dag) DEO(12, true);
       else DEO(12, false);
@@ -139,6 +355,21 @@ void launch_deo(const Geo& g, int nl, int pe, int set, int dag, int clv, int mod
   }
 #undef DEO
 #undef DEO_ARGS
+}
+
+template <typename S>
+void launch_deo(const Geo& g, int nl, int pe, int set, int dag, int clv, int mode, typename Store<S>::R fac, S* out,
+                const S* in, const S* in0, const S* U, const S* C, hipStream_t st) {
+  deo_launch<S, DEO_STORE>(g, nl, pe, set, dag, clv, mode, fac, out, in, in0, U, C, nullptr, nullptr, st);
+}
+
+int deo_reduce_groups(const Geo& g) {
+  return deo_split_pays(g, 0, true) ? deo_split_groups(g) : (int)(((g.V >> 1) + EO_THREADS - 1) / EO_THREADS);
+}
+void launch_deo_reduce(const Geo& g, int pe, int red, double fac, double* out, const double* in, const double* in0,
+                       const double* z, double* part, const double* U, const double* C, hipStream_t st) {
+  if (red == DEO_DOT) deo_launch<double, DEO_DOT>(g, 18, pe, 0, 0, 1, 2, fac, out, in, in0, U, C, z, part, st);
+  else deo_launch<double, DEO_NORM_DOT>(g, 18, pe, 0, 0, 1, 2, fac, out, in, in0, U, C, nullptr, part, st);
 }
 
 // ---------------------------------------------------------------- host layouts

@@ -109,7 +109,9 @@ void launch_update_x(const Batch& B, long long n, R* x, const R* v0, const Scala
 template <typename R>
 void launch_update_p(const Batch& B, long long n, R* p, const R* r, const R* q, const Scalars* sc, hipStream_t st);
 template <typename R> void launch_norm(const Batch& B, long long n, const R* a, double* part, hipStream_t st);
-void launch_finalize(const Batch& B, const double* part, int nval, Scalars* sc, int mode, hipStream_t st);
+// count: partials per value
+void launch_finalize(const Batch& B, const double* part, int nval, Scalars* sc, int mode, hipStream_t st,
+                     int count = RED_BLOCKS);
 // Per-site precision conversion of spinors (V sites; the storage layouts of the
 // precisions differ): out = in / nrm (to lower precision), out = in * nrm (back).
 // so/si: RHS strides of out/in in elements.
@@ -177,6 +179,12 @@ void launch_bqcd(const BqcdGeo& b, int kind, int load, const int* map, double* b
 template <typename S>
 void launch_deo(const Geo& g, int nl, int pe, int set, int dag, int clv, int mode, typename Store<S>::R fac, S* out,
                 const S* in, const S* in0, const S* U, const S* C, hipStream_t st);
+// FP64 out = in0 + fac T^-1 H in on parity pe with sums of out: red DEO_DOT <z, out>,
+// DEO_NORM_DOT |out|^2 and <out, in0>; part[value][deo_reduce_groups(g)]
+enum { DEO_STORE = 0, DEO_DOT = 1, DEO_NORM_DOT = 2 };
+int deo_reduce_groups(const Geo& g);
+void launch_deo_reduce(const Geo& g, int pe, int red, double fac, double* out, const double* in, const double* in0,
+                       const double* z, double* part, const double* U, const double* C, hipStream_t st);
 // kind 0 spinor (one parity), 1 links, 2 clover (both parities); layout 0 plain, 1 QWS AoSoA
 template <typename S>
 void launch_eo_import(const Geo& g, int kind, int layout, int vlen, int nl, const void* src, int src_is_double, S* dst,

@@ -942,18 +942,28 @@ int Lattice::bicgstab_eo(double* x, const double* b, int maxiter, double tol, in
     read_scalars(sc_eo_, 1);
     return std::sqrt(sc_host_[0].rnorm / sc_host_[0].bnorm) < tol;
   };
+  // out = mtilde in with the sums over out that the iteration takes next
+  const int groups = deo_reduce_groups(g_);
+  double* dpart = (double*)work("eob_part", sizeof(double) * 3 * groups);
+  double* t0 = (double*)work("eo_t0", bytes);
+  auto mt = [&](double* out, const double* in, int red) {
+    deo(P64, 1 - pce, 0, 0, 1, 0, 0, t0, in, nullptr);
+    launch_deo_reduce(g_, pce, red, fac, out, t0, in, r0, dpart, Ueo_d_, Ceo_d_, st_);
+  };
   int iter;
   for (iter = 1; iter < maxiter; ++iter) {
-    mtilde(P64, pce, 0, fac, q, p);
-    launch_dot<double>(B, n, r0, q, part, st_);
-    launch_finalize(B, part, 2, sc_eo_, FIN_ALPHA, st_);
-    launch_update_xr<double>(B, n, x, p, r, q, sc_eo_, 0, nullptr, part, st_);
+    mt(q, p, DEO_DOT);
+    launch_finalize(B, dpart, 2, sc_eo_, FIN_ALPHA, st_, groups);
+    // x += alpha p waits for the second half-step's pass over x
+    launch_update_xr<double>(B, n, x, p, r, q, sc_eo_, 0, nullptr, part, st_, XR_R_ONLY);
     launch_finalize(B, part, 1, sc_eo_, FIN_RNORM, st_);
-    if (converged()) break;
-    mtilde(P64, pce, 0, fac, t, r);
-    launch_norm_dot<double>(B, n, t, r, part, st_);
-    launch_finalize(B, part, 3, sc_eo_, FIN_OMEGA, st_);
-    launch_update_xr<double>(B, n, x, r, r, t, sc_eo_, 1, r0, part, st_);
+    if (converged()) {
+      launch_update_x<double>(B, n, x, p, sc_eo_, st_);
+      break;
+    }
+    mt(t, r, DEO_NORM_DOT);
+    launch_finalize(B, dpart, 3, sc_eo_, FIN_OMEGA, st_, groups);
+    launch_update_xr<double>(B, n, x, r, r, t, sc_eo_, 1, r0, part, st_, XR_DEFERRED, p);
     launch_finalize(B, part, 3, sc_eo_, FIN_RHO, st_);
     if (converged()) break;
     launch_update_p<double>(B, n, p, r, q, sc_eo_, st_);

@@ -169,6 +169,50 @@ def test_deo_matches_oracle(eo, set_, dag, clv):
                 assert rel(out.download(), want) < tol, (pe, mode, prec)
 
 
+@pytest.mark.parametrize("L", [[10, 7, 9, 5], [16, 16, 16, 18], [16, 16, 32, 21]])
+def test_deo_around_the_split_rule(L):
+    """Four waves per 64 sites or a thread per site: a ragged last group (1575 sites of a
+    parity), 576 groups (FP64 by threads, FP32 by waves) and 1344 (both by threads)."""
+    rng = np.random.default_rng(19)
+    vh = int(np.prod(L)) // 2
+    U, C = K.random_su3_like(2 * vh, rng)
+    Ue = rng.standard_normal((2, 4, vh, 18))
+    Ce = rng.standard_normal((2, vh, 72)) * 0.1
+    B = [L[0] // 2, L[1], L[2], L[3]]
+    lat = Q.Lattice(L, B, -1, 18, kappa=0.11)
+    lat.eo_load_gauge(Ue)
+    lat.eo_load_clover(Ce)
+    orc = O.Oracle(L, B, -1, 0.11, U, C)
+    a, a0 = rng.standard_normal((vh, 24)), rng.standard_normal((vh, 24))
+    for pe, set_, dag, clv, mode in ((0, 0, False, True, 2), (1, 0, True, False, 1), (0, 2, False, True, 0)):
+        for prec, dt, tol in ((Q.F64, np.float64, 1e-13), (Q.F32, np.float32, 1e-6)):
+            out = lat.eo_spinor(prec, a0)
+            lat.deo(out, lat.eo_spinor(prec, a), pe, set_, dag, clv, mode, -0.37, lat.eo_spinor(prec, a0))
+            want = orc.deo(Ue.astype(dt), Ce.astype(dt), pe, a.astype(dt), set=set_, dag=dag, clv=clv, mode=mode,
+                           fac=dt(-0.37), out=a0.astype(dt).copy(), in0=a0.astype(dt))
+            assert rel(out.download(), want) < tol, (pe, set_, prec)
+
+
+@pytest.mark.parametrize("L", [[8, 4, 4, 8], [12, 16, 12, 32]])
+def test_eo_bicgstab_stops_at_either_half_step(L):
+    """The solve whose sums come with the operator (32 sites to 576 groups of 64: both
+    kernels), stopped at tolerances met by a first or a second half-step: x has every
+    update, the true residual is the tolerance's (FP64 recursion: to 1e-10 of |b| here)."""
+    lat = Q.Lattice(L, [L[0] // 2] + L[1:], -1, 18, kappa=0.115)
+    lat.generate_gauge(0.3, 4)
+    lat.compute_clover(1.0)
+    lat.eo_from_lattice()
+    bh = np.random.default_rng(3).standard_normal((lat.V // 2, 24))
+    b, q = lat.eo_spinor(Q.F64, bh), lat.eo_spinor(Q.F64)
+    its = set()
+    for tol in 10.0 ** -np.arange(1, 9.5, 0.5):
+        x = lat.eo_spinor(Q.F64, np.zeros_like(bh))
+        its.add(lat.eo_bicgstab(x, b, maxiter=200, tol=tol))
+        lat.mtilde(q, x, 0, 0)
+        assert rel(q.download(), bh) < tol * (1 + 1e-6) + 1e-10
+    assert len(its) > 4
+
+
 def test_mtilde_is_schur_complement_of_d():
     """Even extents, fields gathered from the lattice's own: with y_e = x and
     y_o = kappa T_oo^-1 H_oe x, the full D gives (D y)_o = 0 and (D y)_e = mtilde x
