@@ -353,6 +353,7 @@ class Lattice {
   void copy_to_host(void* host, const void* dev, size_t bytes);
   Scalars* sc_h_ = nullptr;     // FP16 SAP input norms, room for MAX_BATCH
   Scalars* sc_eo_ = nullptr;    // even/odd solver
+  hipEvent_t eo_ev_ = nullptr;  // the scalars that bicgstab_eo waits for
   int* d_inner_mask_ = nullptr;
   std::vector<std::pair<std::string, std::pair<void*, size_t>>> work_;
   // while set, work() carves its buffers from this memory instead (prec_ddd_scratch)
