@@ -56,8 +56,25 @@ template <typename S> struct SapMulti {
   int n = 0;
   int xcd = 1;
   int b4 = 0;        // 1: every part has 4^4 blocks (sap4.hip), 0: none has
-  int reserved = 0;  // no padding: launch records are compared by their bytes
+  int rhs = 1;       // grid.y: sap_rhs_groups of the parts' largest nrhs
+                     // (no padding: launch records are compared by their bytes)
 };
+
+// Over how many workgroups the nrhs right-hand sides of a block are spread: a workgroup
+// takes its block's right-hand sides in turn with the links and the clover inverse held,
+// so that a launch on few blocks left most of `slots` (workgroups that run at once) empty.
+// The number with the shortest rounds, in units of one right-hand side; loading the
+// fields is a quarter of one.  12 right-hand sides on 256 blocks (16^3 x 32, nm 6): 313 us with
+// one workgroup per block, 192 with two.
+inline int sap_rhs_groups(int blocks, int nrhs, int slots) {
+  int best = 1;
+  double time = 1e30;
+  for (int k = 1; k <= nrhs; ++k) {
+    const double t = (((long long)blocks * k + slots - 1) / slots) * ((nrhs + k - 1) / k + 0.25);
+    if (t < 0.99 * time) time = t, best = k;
+  }
+  return best;
+}
 
 bool sap_fusable(const Geo& g);
 // 4^4 blocks: the kernels of sap4.hip and sap4h.hip

@@ -200,7 +200,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
   // 1 us each turn), so that one computes while the other waits for memory.  SAP launch,
   // without and with it (nm 6): 4096 blocks 0.316 / 0.308 ms, 2048 blocks 0.170 / 0.162;
   // 512 blocks, a single round, 0.049 / 0.055, so not there.
-  if (gridDim.x >= 1024 && blockIdx.x >= 256 && blockIdx.x < 512)
+  if (gridDim.x >= 1024 && blockIdx.y == 0 && blockIdx.x >= 256 && blockIdx.x < 512)
     for (int i = 6 + nm * 8 / 5; i > 0; --i) __builtin_amdgcn_s_sleep(37);
   const long long first = (long long)blk * VB, site = first + t;
   CloverRegs<float> cl;
@@ -235,7 +235,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
   const int p = lds_pos(t);
   const int epi = flags & SAP_EPI_MASK;
 
-  for (int r = 0; r < nrhs; ++r) {
+  for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
     if (active && !active[r]) continue;  // uniform over the workgroup
     const long long off = r * stride;
     Cx<float> sv[12], acc[12];
@@ -377,9 +377,10 @@ void launch_sap_4444(const Geo& g, BlockSel sel, const Batch& B, int nl, float k
                      const float* in, const float* qface, float* qout, float* out, const float* U, const float* C,
                      float* fb, long long fbs, hipStream_t st, const SapSrcUpdate& upd) {
 #define SAP4(NL, FB)                                                                                              \
-  hipLaunchKernelGGL((k_sap_4444<NL, FB, false>), dim3(sel.n), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, \
+  hipLaunchKernelGGL((k_sap_4444<NL, FB, false>), dim3(sel.n, ny), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, \
                      kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, upd, SapMulti<float>())
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
+  const int ny = sap_rhs_groups(sel.n, B.n, 512);
   if (nl == 12) {
     if (fbk) SAP4(12, true);
     else SAP4(12, false);
@@ -394,7 +395,7 @@ void launch_sap_4444_multi(const SapMulti<float>& m, int nl, int nm, int flags, 
   const Geo g0{};
   const SapSrcUpdate u0;
 #define SAP4(NL, FB)                                                                                               \
-  hipLaunchKernelGGL((k_sap_4444<NL, FB, true>), dim3(m.n), dim3(VB), 0, st, g0, nullptr, 0, 0, nullptr, 0.0f, nm, flags, \
+  hipLaunchKernelGGL((k_sap_4444<NL, FB, true>), dim3(m.n, m.rhs), dim3(VB), 0, st, g0, nullptr, 0, 0, nullptr, 0.0f, nm, flags, \
                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, u0, m)
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
   if (nl == 12) {

@@ -283,7 +283,7 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
   const int p = lds_pos(t);
   const int epi = flags & SAP_EPI_MASK;
 
-  for (int r = 0; r < nrhs; ++r) {
+  for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
     if (active && !active[r]) continue;  // uniform over the workgroup
     const long long off = r * stride;
     h2v sv[12];
@@ -408,9 +408,10 @@ void launch_sap_4444_h(const Geo& g, BlockSel sel, const Batch& B, int nl, float
                        const __half* in, const __half* qface, __half* qout, __half* out, const __half* U, const __half* C,
                        float* fb, long long fbs, hipStream_t st) {
 #define SAP4H(NL, FB)                                                                                                  \
-  hipLaunchKernelGGL((k_sap_4444_h<NL, FB>), dim3(sel.n), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, kappa, \
+  hipLaunchKernelGGL((k_sap_4444_h<NL, FB>), dim3(sel.n, ny), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, kappa, \
                      nm, flags, s, in, qface, qout, out, U, C, fb, fbs)
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
+  const int ny = sap_rhs_groups(sel.n, B.n, 512);
   if (nl == 12) {
     if (fbk) SAP4H(12, true);
     else SAP4H(12, false);

@@ -44,6 +44,25 @@ def test_batch_equals_single_bitwise(lat):
         assert st[k]["true_residual"] <= 1e-10
 
 
+@pytest.mark.parametrize("L,B,n,sap", [([16, 16, 16, 32], [4, 4, 4, 4], 5, Q.F32), ([16, 16, 16, 32], [4, 4, 4, 4], 3, Q.F16),
+                                       ([24, 16, 16, 32], [4, 4, 4, 4], 4, Q.F32), ([16, 8, 8, 8], [8, 4, 4, 4], 4, Q.F32)])
+def test_right_hand_sides_spread_over_workgroups(L, B, n, sap):
+    """256 and 384 blocks per colour, 8 of 512 sites: a block's right-hand sides go to two
+    workgroups (3 and 2, or 2 and 1 of them), to four or to one each, with the others'
+    result bit for bit that of a solve alone."""
+    lat = Q.Lattice(L, B, -1, 12, kappa=0.12)
+    lat.generate_gauge(0.3, 12)
+    lat.compute_clover(1.0)
+    bs = _sources(lat, n)
+    xs = [lat.spinor(Q.F64) for _ in range(n)]
+    prm = dict(PRM, nsap=3 if sap == Q.F16 else 2, nm=3, maxiter=2, max_restarts=0, sap_precision=sap)
+    lat.solve_batch(xs, bs, **prm)
+    for k in range(n):
+        x1 = lat.spinor(Q.F64)
+        lat.solve(x1, bs[k], **prm)
+        assert x1.digest() == xs[k].digest(), k
+
+
 def test_batch_with_initial_guess_and_oracle_residual(lat):
     n = 3
     bs = _sources(lat, n)
