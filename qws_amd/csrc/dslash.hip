@@ -78,21 +78,35 @@ k_hop(Geo g, const int* __restrict__ list, int wg_per_blk, int nrhs, long long s
   }
 }
 
-// Full operator out = in + gamma T^-1 H in for one right-hand side over every
-// site: the kernel for D itself (ddd_d_, ddd_s_ and the outer solver's D).  Written
-// without the generality of k_hop (RHS loop, a/b/c terms, block lists) it keeps the
-// live state of a thread small (about 90 VGPRs in FP32).  It is compiled for at most
+// The right-hand side of logical workgroup wg of a full operator, by its offset in the
+// spinors, and in wg the workgroup of its blocks; false where it is not active.  Those
+// of one block are neighbours, on one XCD, so that the links and the clover inverse come
+// from its L2 for all but the first (12 right-hand sides on 16^3 x 32, FP64, one after
+// another / so: 680 / 393 us).
+__device__ __forceinline__ bool rhs_of(int& wg, int nrhs, long long stride, const int* active, long long& off) {
+  const int r = nrhs == 1 ? 0 : wg % nrhs;
+  if (nrhs != 1) wg /= nrhs;
+  off = r * stride;
+  return !(active && !active[r]);
+}
+
+// Full operator out = in + gamma T^-1 H in over every site: the kernel for D itself
+// (ddd_d_, ddd_s_ and the outer solver's D).  Written without the generality of k_hop
+// (RHS loop, a/b/c terms, block lists) it keeps the live state of a thread small (about
+// 90 VGPRs in FP32).  It is compiled for at most
 // 3 waves per SIMD (amdgpu_waves_per_eu): the schedule that results orders the
 // neighbour gathers so that FP32 32^3x64 fetches 1.3x less from HBM than the default
 // schedule and runs 2% faster (the register count still admits 5 waves per SIMD).
 template <typename S, int NL, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, 3)))
-k_dslash(Geo g, const int* __restrict__ order, int wg_per_blk, const int* __restrict__ active,
-         typename Store<S>::R gamma, S* __restrict__ out, const S* __restrict__ in, const S* __restrict__ U,
-         const S* __restrict__ C) {
+k_dslash(Geo g, const int* __restrict__ order, int wg_per_blk, int nrhs, long long stride,
+         const int* __restrict__ active, typename Store<S>::R gamma, S* __restrict__ out, const S* __restrict__ in,
+         const S* __restrict__ U, const S* __restrict__ C) {
   using R = typename Store<S>::R;
-  if (active && !*active) return;
-  const int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  long long off;
+  if (!rhs_of(wg, nrhs, stride, active, off)) return;
+  in += off, out += off;
   const int bi = wg / wg_per_blk;
   const int loc = (wg - bi * wg_per_blk) * HOP_THREADS + threadIdx.x;
   if (loc >= g.Vb) return;
@@ -151,12 +165,15 @@ __device__ __forceinline__ void hop_staged(const Geo& g, long long s, const Site
 // (Nontemporal link and clover loads were measured slower here, with more L2 misses.)
 template <int NL, int W, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, W)))
-k_dslash_lds(Geo g, const int* __restrict__ order, const int* __restrict__ active, float gamma, float* __restrict__ out,
+k_dslash_lds(Geo g, const int* __restrict__ order, int nrhs, long long stride, const int* __restrict__ active, float gamma, float* __restrict__ out,
              const float* __restrict__ in, const float* __restrict__ U, const float* __restrict__ C) {
   __shared__ float4 lx[6 * HOP_THREADS];
-  if (active && !*active) return;
+  int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  long long off;
+  if (!rhs_of(wg, nrhs, stride, active, off)) return;
+  in += off, out += off;
   const int t = threadIdx.x;
-  const long long s = (long long)order[xcd_remap(g, blockIdx.x, gridDim.x)] * HOP_THREADS + t;
+  const long long s = (long long)order[wg] * HOP_THREADS + t;
   const float4* iv = reinterpret_cast<const float4*>(in);
 #pragma unroll
   for (int j = 0; j < 6; ++j) lx[j * HOP_THREADS + t] = iv[(long long)j * g.V + s];
@@ -185,11 +202,11 @@ k_dslash_lds(Geo g, const int* __restrict__ order, const int* __restrict__ activ
 }
 
 template <int NL>
-void launch_dslash_lds(const Geo& g, BlockSel sel, const int* active, float gamma, float* out, const float* in,
+void launch_dslash_lds(const Geo& g, BlockSel sel, const Batch& B, bool nt, float gamma, float* out, const float* in,
                        const float* U, const float* C, hipStream_t st) {
-  const bool nt = operator_bytes<float>(g, NL) > DSLASH_STREAM_BYTES;
-#define DSL_LDS(W, NT) \
-  hipLaunchKernelGGL((k_dslash_lds<NL, W, NT>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, active, gamma, out, in, U, C)
+#define DSL_LDS(W, NT)                                                                                             \
+  hipLaunchKernelGGL((k_dslash_lds<NL, W, NT>), dim3(sel.n * B.n), dim3(HOP_THREADS), 0, st, g, sel.list, B.n, B.stride, \
+                     B.active, gamma, out, in, U, C)
   if (g.dslash_kernel == 3) {
     if (nt) DSL_LDS(3, true);
     else DSL_LDS(3, false);
@@ -234,13 +251,16 @@ __device__ __forceinline__ void hop_staged_d(const Geo& g, long long s, const Si
 // spinor staged in LDS (12 double2 planes, 48 KB): bit for bit k_dslash<double, 18>.
 template <int W, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, W)))
-k_dslash_lds_d(Geo g, const int* __restrict__ order, const int* __restrict__ active, double gamma,
+k_dslash_lds_d(Geo g, const int* __restrict__ order, int nrhs, long long stride, const int* __restrict__ active, double gamma,
                double* __restrict__ out, const double* __restrict__ in, const double* __restrict__ U,
                const double* __restrict__ C) {
   __shared__ double2 lx[12 * HOP_THREADS];
-  if (active && !*active) return;
+  int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  long long off;
+  if (!rhs_of(wg, nrhs, stride, active, off)) return;
+  in += off, out += off;
   const int t = threadIdx.x;
-  const long long s = (long long)order[xcd_remap(g, blockIdx.x, gridDim.x)] * HOP_THREADS + t;
+  const long long s = (long long)order[wg] * HOP_THREADS + t;
   const double2* iv = reinterpret_cast<const double2*>(in);
 #pragma unroll
   for (int k = 0; k < 12; ++k) lx[k * HOP_THREADS + t] = iv[(long long)k * g.V + s];
@@ -277,43 +297,36 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
     return;
   }
   if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
-    // the full operator: one lean launch per right-hand side
-    const bool nt = operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
+    // the full operator (several right-hand sides share their clover through the caches)
+    const bool nt = B.n == 1 && operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
     if constexpr (std::is_same<S, float>::value) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel != 0) {
-        for (int r = 0; r < B.n; ++r)
-          launch_dslash_lds<NL>(g, sel, B.active ? B.active + r : nullptr, gamma, out + r * B.stride,
-                                in + r * B.stride, U, C, st);
+        launch_dslash_lds<NL>(g, sel, B, nt, gamma, out, in, U, C, st);
         return;
       }
     }
     if constexpr (std::is_same<S, double>::value && NL == 18) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel_d != 0) {
-        for (int r = 0; r < B.n; ++r) {
-          const int* act = B.active ? B.active + r : nullptr;
-#define DSL_LDS(W, NT)                                                                                           \
-  hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n), dim3(HOP_THREADS), 0, st, g, sel.list, act, gamma, \
-                     out + r * B.stride, in + r * B.stride, U, C)
-          if (g.dslash_kernel_d == 2) {
-            if (nt) DSL_LDS(2, true);
-            else DSL_LDS(2, false);
-          } else {
-            if (nt) DSL_LDS(3, true);
-            else DSL_LDS(3, false);
-          }
-#undef DSL_LDS
+#define DSL_LDS(W, NT)                                                                                          \
+  hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n * B.n), dim3(HOP_THREADS), 0, st, g, sel.list, B.n, B.stride, \
+                     B.active, gamma, out, in, U, C)
+        if (g.dslash_kernel_d == 2) {
+          if (nt) DSL_LDS(2, true);
+          else DSL_LDS(2, false);
+        } else {
+          if (nt) DSL_LDS(3, true);
+          else DSL_LDS(3, false);
         }
+#undef DSL_LDS
         return;
       }
     }
     const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
-#define DSL(NT)                                                                                         \
-  hipLaunchKernelGGL((k_dslash<S, NL, NT>), dim3(sel.n * wpb), dim3(HOP_THREADS), 0, st, g, sel.list, wpb, \
-                     B.active ? B.active + r : nullptr, gamma, out + r * B.stride, in + r * B.stride, U, C)
-    for (int r = 0; r < B.n; ++r) {
-      if (nt) DSL(true);
-      else DSL(false);
-    }
+#define DSL(NT)                                                                                                  \
+  hipLaunchKernelGGL((k_dslash<S, NL, NT>), dim3(sel.n * wpb * B.n), dim3(HOP_THREADS), 0, st, g, sel.list, wpb, B.n, \
+                     B.stride, B.active, gamma, out, in, U, C)
+    if (nt) DSL(true);
+    else DSL(false);
 #undef DSL
     return;
   }
