@@ -23,6 +23,15 @@ constexpr int HOP_THREADS = 256;
 //   340 MB  77.3 / 69.0    446 MB   108 / 88.9   1409 MB   337 / 313     FP64 1019 MB 253 / 235
 constexpr double DSLASH_STREAM_BYTES = 280e6;
 
+// Blocks that an XCD takes in turn in the LDS-staged full operators (xcd_chunk), in index
+// order.  With a contiguous eighth of the lattice for each XCD every face that its L2 has
+// lost comes from memory; side by side the XCDs find it in the last-level cache.  us, a
+// contiguous range / chunks of 8 / of 64:
+//   FP64  24^3 48 234 / 214 / 221   32^4 364 / 353 / 348   40 24 32 40 444 / 404 / 412   32^3 64 768 / 681 / 721
+//   FP32  24^3 48  94 /  93 /  93   32^4 152 / 158 / 150   40 24 32 40 187 / 178 / 179   32^3 64 321 / 310 / 313
+// (No gain for k_dslash on large blocks, nor for the even/odd operator.)
+constexpr int DSLASH_CHUNK_64 = 8, DSLASH_CHUNK_32 = 64;
+
 template <typename S, int NL, int SET>
 __global__ void __launch_bounds__(HOP_THREADS)
 k_hop(Geo g, const int* __restrict__ list, int wg_per_blk, int nrhs, long long stride, const int* __restrict__ active,
@@ -289,7 +298,7 @@ k_dslash_lds_d(Geo g, const int* __restrict__ order, int nrhs, long long stride,
 
 template <typename S, int NL>
 void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a,
-                const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st) {
+                const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st, bool index_order) {
   if (split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value)) {
     SplitPart<S> p;
     p.sel = sel, p.set = set, p.gamma = gamma, p.out = out, p.a = a, p.b = b, p.c = c, p.in = in;
@@ -298,17 +307,19 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
   }
   if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
     // the full operator (several right-hand sides share their clover through the caches)
+    Geo gc = g;
+    if (index_order && B.n == 1) gc.xcd_chunk = sizeof(S) == 8 ? DSLASH_CHUNK_64 : DSLASH_CHUNK_32;
     const bool nt = B.n == 1 && operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
     if constexpr (std::is_same<S, float>::value) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel != 0) {
-        launch_dslash_lds<NL>(g, sel, B, nt, gamma, out, in, U, C, st);
+        launch_dslash_lds<NL>(gc, sel, B, nt, gamma, out, in, U, C, st);
         return;
       }
     }
     if constexpr (std::is_same<S, double>::value && NL == 18) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel_d != 0) {
 #define DSL_LDS(W, NT)                                                                                          \
-  hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n * B.n), dim3(HOP_THREADS), 0, st, g, sel.list, B.n, B.stride, \
+  hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n * B.n), dim3(HOP_THREADS), 0, st, gc, sel.list, B.n, B.stride, \
                      B.active, gamma, out, in, U, C)
         if (g.dslash_kernel_d == 2) {
           if (nt) DSL_LDS(2, true);
@@ -352,7 +363,7 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
 
 #define INST_HOP(S, NL)                                                                                           \
   template void launch_hop<S, NL>(const Geo&, BlockSel, const Batch&, int, typename Store<S>::R, S*, const S*,     \
-                                  const S*, const S*, const S*, const S*, const S*, hipStream_t);
+                                  const S*, const S*, const S*, const S*, const S*, hipStream_t, bool);
 INST_HOP(float, 18)
 INST_HOP(float, 12)
 INST_HOP(double, 18)

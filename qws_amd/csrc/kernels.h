@@ -20,11 +20,12 @@ struct BlockSel {
 // out = a + b - c + gamma * T^-1 H_set(in)  on the selected blocks.
 // Any of a, b, c may be nullptr (term absent).  out may alias a, b or c, never in.
 // skip_interior: for set == HOPS_FACE with out == a, sites without a face hop
-// are left untouched.
+// are left untouched.  index_order: the list is every block, in index order.
 struct Batch;
 template <typename S, int NL>
 void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a,
-                const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st);
+                const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st,
+                bool index_order = false);
 
 // One operator of launch_split: the arguments of launch_hop (a face hop set with out == a
 // alone leaves the sites without a face hop untouched) and the hops it may take, all or

@@ -75,6 +75,7 @@ Lattice::Lattice(const int L[4], const int B[4], int tbc, int links32) {
   g_.V = V;
   g_.tbc = tbc;
   g_.hopmask = 0xFF;
+  g_.xcd_chunk = 0;
   // workgroup placement: XCD-contiguous block ranges unless QWS_MI355X_XCD_REMAP=0
   const char* xr = std::getenv("QWS_MI355X_XCD_REMAP");
   g_.xcd_remap = (xr && xr[0] == '0') ? 0 : 1;
@@ -441,9 +442,10 @@ void Lattice::hop(BlockSel s, const Batch& B, int set, typename Store<S>::R gamm
                   const S* c, const S* in) {
   if (s.n == 0) return;
   FieldSet<S> f = fields<S>();
-  if (f.nl == 18) launch_hop<S, 18>(g_, s, B, set, gamma, out, a, b, c, in, f.U, f.C, st_);
+  const bool io = s.list == d_order_;
+  if (f.nl == 18) launch_hop<S, 18>(g_, s, B, set, gamma, out, a, b, c, in, f.U, f.C, st_, io);
   else if constexpr (!std::is_same<S, double>::value)
-    launch_hop<S, 12>(g_, s, B, set, gamma, out, a, b, c, in, f.U, f.C, st_);
+    launch_hop<S, 12>(g_, s, B, set, gamma, out, a, b, c, in, f.U, f.C, st_, io);
 }
 
 // Two operators that do not depend on each other: one launch where few sites are at work.

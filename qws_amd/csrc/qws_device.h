@@ -43,6 +43,7 @@ struct Geo {
                   // runtime value it keeps each hop in its own basic block, so the
                   // compiler cannot hoist all eight neighbour loads (256 -> ~146 VGPRs)
   int xcd_remap;  // 1: map workgroups to blocks XCD by XCD (xcd_remap), 0: identity
+  int xcd_chunk;  // 0: a contiguous range for each XCD, else chunks of so many workgroups in turn
   int dslash_kernel;  // FP32 full operator on 256-site blocks: 0 global gathers (k_dslash),
                       // 3/4: block spinor staged in LDS, compiled for that many waves per SIMD
   int dslash_kernel_d;  // the same for FP64 (18-real links): 0 gathers, 2/3 LDS-staged
@@ -50,15 +51,23 @@ struct Geo {
 
 // MI355X dispatches the workgroups of a launch round-robin over its 8 XCDs, each
 // with its own L2.  Give XCD x a contiguous range of logical workgroup ids (blocks
-// that share faces then share an L2): a bijection of [0, nwg).
+// that share faces then share an L2), or with chunk > 0 every eighth chunk of so many:
+// the XCDs then go through the lattice side by side, and what one fetches another
+// finds in the last-level cache.  A bijection of [0, nwg).
 constexpr int NUM_XCD = 8;
-__device__ __forceinline__ int xcd_remap_n(int on, int wg, int nwg) {
+__device__ __forceinline__ int xcd_remap_n(int on, int wg, int nwg, int chunk = 0) {
   if (!on) return wg;
-  const int q = nwg / NUM_XCD, r = nwg % NUM_XCD;
   const int x = wg % NUM_XCD, i = wg / NUM_XCD;
+  if (chunk > 0) {
+    const int whole = nwg - nwg % (NUM_XCD * chunk);
+    return wg < whole ? (i / chunk * NUM_XCD + x) * chunk + i % chunk : wg;
+  }
+  const int q = nwg / NUM_XCD, r = nwg % NUM_XCD;
   return x * q + (x < r ? x : r) + i;
 }
-__device__ __forceinline__ int xcd_remap(const Geo& g, int wg, int nwg) { return xcd_remap_n(g.xcd_remap, wg, nwg); }
+__device__ __forceinline__ int xcd_remap(const Geo& g, int wg, int nwg) {
+  return xcd_remap_n(g.xcd_remap, wg, nwg, g.xcd_chunk);
+}
 
 // p, hidden from the optimiser.  Loads through the result taken inside a loop over
 // right-hand sides are not loop-invariant to the compiler, so it does not hoist a
