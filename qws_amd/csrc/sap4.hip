@@ -16,6 +16,7 @@
 // Bound by the latency of a Jacobi step: two waves per SIMD, four barriers, 975 vector
 // instructions per wave in 7400 cycles, as long with one workgroup on the CU as with two.
 // More waves do not fit: links, clover, source and sum take 251 of 256 registers.
+// (Launches on few blocks have a CU for each: WIDE takes eight waves.)
 // A launch on 4096 blocks (half of 32^3 x 64; nm 6), general kernel / this one: 12-real links
 // 0.335 / 0.306 ms, 18-real (which the general kernel reads from memory at each hop)
 // 0.564 / 0.314 ms; on 8 blocks (8^4) 0.0316 / 0.0285 ms.
@@ -137,6 +138,55 @@ __device__ __forceinline__ void block_hops(const f4v* lx, f4v* lh, int wave, int
   if (l.t > 0) add_half<3, -1>(hs, 2.0f, acc);
 }
 
+// The same with the backward tasks on four more waves at the same time (helper), into half
+// spinors of their own.
+__device__ __forceinline__ void block_hops_wide(const f4v* lx, f4v* lh, int wave, int p, const WaveLinks& w,
+                                                Cx<float> acc[12]) {
+  Raw r;
+  Halves hs;
+  const Coord l = coord(threadIdx.x, wave);
+  __syncthreads();
+  if (wave < 3) {
+    read_raw<0, +1>(lx, from<+1>(w, 0), r);
+    tasks<0, 1, 2, +1>(lx, lh, w, r);
+    asm volatile("; x y z");
+  } else {
+    read_raw<3, +1>(lx, from<+1>(w, 0), r);
+    tasks<3, 3, 3, +1>(lx, lh, w, r);
+    asm volatile("; t");
+  }
+  __syncthreads();
+  read_halves(lh, p, hs);
+  fence();
+#pragma unroll
+  for (int k = 0; k < 12; ++k) acc[k] = {0, 0};
+  if (l.x < 3) add_half<0, +1>(hs, 2.0f, acc);
+  if (l.y < 3) add_half<1, +1>(hs, 2.0f, acc);
+  if (l.z < 3) add_half<2, +1>(hs, 2.0f, acc);
+  if (l.t < 3) add_half<3, +1>(hs, 2.0f, acc);
+  fence();
+  read_halves(lh + 12 * VB, p, hs);
+  fence();
+  if (l.x > 0) add_half<0, -1>(hs, 2.0f, acc);
+  if (l.y > 0) add_half<1, -1>(hs, 2.0f, acc);
+  if (l.z > 0) add_half<2, -1>(hs, 2.0f, acc);
+  if (l.t > 0) add_half<3, -1>(hs, 2.0f, acc);
+}
+__device__ __forceinline__ void helper(const f4v* lx, f4v* lh, int wave, const WaveLinks& w) {
+  Raw r;
+  __syncthreads();
+  if (wave < 3) {
+    read_raw<0, -1>(lx, from<-1>(w, 0), r);
+    tasks<0, 1, 2, -1>(lx, lh + 12 * VB, w, r);
+    asm volatile("; x y z");
+  } else {
+    read_raw<3, -1>(lx, from<-1>(w, 0), r);
+    tasks<3, 3, 3, -1>(lx, lh + 12 * VB, w, r);
+    asm volatile("; t");
+  }
+  __syncthreads();
+}
+
 // The block's site t of a spinor field: uniform base, 32-bit lane offset (no 64-bit
 // address per plane in vector registers).
 __device__ __forceinline__ void load_site(const float* f, long long first, long long V, unsigned t, Cx<float> v[12]) {
@@ -170,20 +220,21 @@ __device__ __forceinline__ void face_produce(const f4v* lx, int j, int p3, int p
 }
 
 // The arguments and steps of k_sap_block (sap_kernels.inc); FB: face updates through the
-// face buffer, else by gathers, both with the same roundings.
-template <int NL, bool FB, bool MULTI>
-__global__ void __launch_bounds__(VB, 2)
+// face buffer, else by gathers, both with the same roundings.  WIDE: 512 threads, waves 4
+// to 7 for the backward tasks, one workgroup per CU (123 KB of LDS); bit for bit the same.
+template <int NL, bool FB, bool MULTI, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 2 * VB : VB, 2)
 k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, const int* __restrict__ active, float kappa,
            int nm, int flags, float* s, const float* in, const float* qface, float* qout, float* out,
            const float* __restrict__ U, const float* __restrict__ C, float* fb, long long fbs, SapSrcUpdate upd,
            SapMulti<float> multi) {
   constexpr int NC = NL / 2;
-  __shared__ f4v sm[(6 + 12) * VB];
+  __shared__ f4v sm[(6 + (WIDE ? 24 : 12)) * VB];
   f4v* lx = sm;           // the iterate, float4 [6][VB]
-  f4v* lh = sm + 6 * VB;  // half spinors, float4 [4][3][VB]
+  f4v* lh = sm + 6 * VB;  // half spinors, float4 [4][3][VB] (WIDE: of each direction)
   const unsigned t = threadIdx.x;
   const int j = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wave8 = __builtin_amdgcn_readfirstlane(t >> 6), wave = wave8 & 3;
   int blk;
   if constexpr (MULTI) {
     const int2 e = multi.table[xcd_remap_n(multi.xcd, blockIdx.x, gridDim.x)];
@@ -204,7 +255,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
     for (int i = 6 + nm * 8 / 5; i > 0; --i) __builtin_amdgcn_s_sleep(37);
   const long long first = (long long)blk * VB, site = first + t;
   CloverRegs<float> cl;
-  cl.load(C, site, g.V);
+  if (!WIDE || wave8 < 4) cl.load(C, site, g.V);
 
   WaveLinks wl;
 #pragma unroll
@@ -215,6 +266,22 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
     wl.pn[i] = lds_pos(ls + (1 << (2 * mu)));
 #pragma unroll
     for (int k = 0; k < NC; ++k) wl.u[i][k] = load_cx<float>(U + 2 * (((long long)mu * NC + k) * g.V + first), ls);
+  }
+  const int epi = flags & SAP_EPI_MASK;
+  if (WIDE && wave8 >= 4) {  // (the barriers of the other waves' way through the loop below)
+    if (NL == 12) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) link_row2(wl.u[i]);
+    }
+    for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
+      if (active && !active[r]) continue;
+      __syncthreads();
+      if (FB && (flags & SAP_FACE_PRO)) __syncthreads();
+      for (int it = 0; it < nm; ++it) helper(lx, lh, wave, wl);
+      if (epi != SAP_EPI_NONE) helper(lx, lh, wave, wl);
+      else __syncthreads();
+    }
+    return;
   }
   // the wave's face links, loaded where they are used (they are in cache, and there are
   // no registers to keep them in during the block solve)
@@ -233,12 +300,15 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
   }
   const float tf_hi = b[3] == g.NB[3] - 1 ? 2.0f * g.tbc : 2.0f, tf_lo = b[3] == 0 ? 2.0f * g.tbc : 2.0f;
   const int p = lds_pos(t);
-  const int epi = flags & SAP_EPI_MASK;
 
   for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
     if (active && !active[r]) continue;  // uniform over the workgroup
     const long long off = r * stride;
     Cx<float> sv[12], acc[12];
+    auto hops = [&]() {
+      if (WIDE) block_hops_wide(lx, lh, wave, p, wl, acc);
+      else block_hops(lx, lh, wave, p, wl, acc);
+    };
     if (flags & SAP_SRC_PUPD) src_update(upd, r, off, opaque_v(site), g.V);
     // every load of the prologue is issued here, with those of the links and the clover
     // still on their way (one round trip to memory, not three)
@@ -296,7 +366,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
     }
     fence();
     for (int it = 0; it < nm; ++it) {
-      block_hops(lx, lh, wave, p, wl, acc);
+      hops();
       fence();
       clover_regs(cl, acc);
 #pragma unroll
@@ -312,7 +382,7 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
 
     if (epi != SAP_EPI_NONE) {
       // acc = T^-1 H_in x
-      block_hops(lx, lh, wave, p, wl, acc);
+      hops();
       const unsigned te = fresh_thread();
       // (SAP_EPI_OUT takes nothing: one line of s for all threads, so that the loads need no branch)
       const float* src = epi == SAP_EPI_SUPDATE || (flags & SAP_SRC_IN) ? in : s;
@@ -371,40 +441,60 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
 
 }  // namespace
 
+// At most that many workgroups, a quarter of the CUs: the wide kernel.  It takes a CU for
+// itself, so that launches of other streams have to find theirs.  us, the other / it: 8 blocks
+// (8^4) nm 2 16.7 / 14.6, nm 6 29.2 / 23.5; 64 blocks nm 6 31.6 / 26.1; 256 blocks nm 6 alone 34.8
+// / 29.8, but nm 2 on three streams at once 11.7 / 17.5 a launch.
+constexpr int WIDE_GROUPS = 64;
+
 bool sap_is_4444(const Geo& g) { return g.B[0] == 4 && g.B[1] == 4 && g.B[2] == 4 && g.B[3] == 4; }
 
 void launch_sap_4444(const Geo& g, BlockSel sel, const Batch& B, int nl, float kappa, int nm, int flags, float* s,
                      const float* in, const float* qface, float* qout, float* out, const float* U, const float* C,
                      float* fb, long long fbs, hipStream_t st, const SapSrcUpdate& upd) {
-#define SAP4(NL, FB)                                                                                              \
-  hipLaunchKernelGGL((k_sap_4444<NL, FB, false>), dim3(sel.n, ny), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, \
+#define SAP4(NL, FB, WIDE)                                                                                              \
+  hipLaunchKernelGGL((k_sap_4444<NL, FB, false, WIDE>), dim3(sel.n, ny), dim3(WIDE ? 2 * VB : VB), 0, st, g, sel.list, B.n, B.stride, B.active, \
                      kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs, upd, SapMulti<float>())
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
   const int ny = sap_rhs_groups(sel.n, B.n, 512);
+  const bool wide = sel.n * ny <= WIDE_GROUPS;
+#define SAP4W(NL, FB)             \
+  do {                            \
+    if (wide) SAP4(NL, FB, true); \
+    else SAP4(NL, FB, false);     \
+  } while (0)
   if (nl == 12) {
-    if (fbk) SAP4(12, true);
-    else SAP4(12, false);
+    if (fbk) SAP4W(12, true);
+    else SAP4W(12, false);
   } else {
-    if (fbk) SAP4(18, true);
-    else SAP4(18, false);
+    if (fbk) SAP4W(18, true);
+    else SAP4W(18, false);
   }
+#undef SAP4W
 #undef SAP4
 }
 
 void launch_sap_4444_multi(const SapMulti<float>& m, int nl, int nm, int flags, hipStream_t st) {
   const Geo g0{};
   const SapSrcUpdate u0;
-#define SAP4(NL, FB)                                                                                               \
-  hipLaunchKernelGGL((k_sap_4444<NL, FB, true>), dim3(m.n, m.rhs), dim3(VB), 0, st, g0, nullptr, 0, 0, nullptr, 0.0f, nm, flags, \
+#define SAP4(NL, FB, WIDE)                                                                                               \
+  hipLaunchKernelGGL((k_sap_4444<NL, FB, true, WIDE>), dim3(m.n, m.rhs), dim3(WIDE ? 2 * VB : VB), 0, st, g0, nullptr, 0, 0, nullptr, 0.0f, nm, flags, \
                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, u0, m)
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
+  const bool wide = m.n * m.rhs <= WIDE_GROUPS;
+#define SAP4W(NL, FB)             \
+  do {                            \
+    if (wide) SAP4(NL, FB, true); \
+    else SAP4(NL, FB, false);     \
+  } while (0)
   if (nl == 12) {
-    if (fbk) SAP4(12, true);
-    else SAP4(12, false);
+    if (fbk) SAP4W(12, true);
+    else SAP4W(12, false);
   } else {
-    if (fbk) SAP4(18, true);
-    else SAP4(18, false);
+    if (fbk) SAP4W(18, true);
+    else SAP4W(18, false);
   }
+#undef SAP4W
 #undef SAP4
 }
 

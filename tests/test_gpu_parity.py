@@ -261,11 +261,12 @@ def test_fused_sap_face_buffer_is_bitwise_the_gather(L, B, su3, nsap, nm):
 
 @pytest.mark.parametrize("su3", [True, False])
 @pytest.mark.parametrize("L,nsap,nm", [([8, 8, 8, 8], 1, 1), ([8, 8, 8, 8], 3, 2), ([24, 8, 16, 8], 2, 1),
-                                       ([24, 8, 16, 8], 0, 5), ([32, 16, 32, 32], 1, 2)])
+                                       ([24, 8, 16, 8], 0, 5), ([24, 8, 16, 16], 2, 2), ([32, 16, 32, 32], 1, 2)])
 def test_fused_sap_4444(L, nsap, nm, su3):
     """The FP32 kernel for 4^4 blocks (hops by link, not by site) where both neighbours
     of a block are the same one, at extents that differ in every direction, with one Jacobi
-    step, with 12- and 18-real links, and on 1024 blocks per colour (second workgroups
+    step, with 12- and 18-real links, by eight waves a block (to 64 blocks per colour, here
+    8 and 48) and by four (96), and on 1024 blocks per colour (second workgroups
     start late): the oracle's result, by the face buffer bit for bit as by gathers.  On the
     largest lattice against the step-by-step kernels.  FP32 rounding: 1e-6 at most over
     the few hundred operations behind a component, 5e-6 allowed as in the tests above."""
