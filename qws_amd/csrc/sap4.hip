@@ -441,12 +441,6 @@ k_sap_4444(Geo g, const int* __restrict__ list, int nrhs, long long stride, cons
 
 }  // namespace
 
-// At most that many workgroups, a quarter of the CUs: the wide kernel.  It takes a CU for
-// itself, so that launches of other streams have to find theirs.  us, the other / it: 8 blocks
-// (8^4) nm 2 16.7 / 14.6, nm 6 29.2 / 23.5; 64 blocks nm 6 31.6 / 26.1; 256 blocks nm 6 alone 34.8
-// / 29.8, but nm 2 on three streams at once 11.7 / 17.5 a launch.
-constexpr int WIDE_GROUPS = 64;
-
 bool sap_is_4444(const Geo& g) { return g.B[0] == 4 && g.B[1] == 4 && g.B[2] == 4 && g.B[3] == 4; }
 
 void launch_sap_4444(const Geo& g, BlockSel sel, const Batch& B, int nl, float kappa, int nm, int flags, float* s,

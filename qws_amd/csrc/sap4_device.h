@@ -12,6 +12,13 @@ namespace sap4 {
 constexpr int VB = 256;  // sites per block = threads per workgroup
 constexpr int FS = 512;  // face slots per block (sap_kernels.inc has their order)
 
+// At most that many workgroups, a quarter of the CUs: the wide kernel.  It takes a CU for
+// itself, so that launches of other streams have to find theirs.  us, the other / it: 8 blocks
+// (8^4) nm 2 16.7 / 14.6, nm 6 29.2 / 23.5; 64 blocks nm 6 31.6 / 26.1; 256 blocks nm 6 alone 34.8
+// / 29.8, but nm 2 on three streams at once 11.7 / 17.5 a launch  FP16: 8 blocks nm 2 15.6 /
+// 14.1, nm 6 26.3 / 22.7.
+constexpr int WIDE_GROUPS = 64;
+
 // Position of block site s = (x, y, z, t) in an LDS plane of float4: its low four bits
 // (x, y) XORed by a constant for each z.  A 128-bit LDS read serves lanes 0-3, 12-15 and
 // 20-27 (then the others of 32) at once from 16 groups of 16 bytes, a write eight lanes in

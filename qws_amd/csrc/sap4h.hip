@@ -93,8 +93,17 @@ template <int DIR> __device__ __forceinline__ void t_task(const h2v u[9], const 
   link_mult_h2<DIR>(u, a, h);
   reconstruct<float, 3, DIR>(h, 2.0f, acc);
 }
-template <int W, int DIR>
-__device__ __forceinline__ void wave_tasks(const f4v* lx, f4v* lh, int p, const WaveLinks& w, Raw& r, Cx<float> acc[12]) {
+template <int DIR> __device__ __forceinline__ void t_task_lds(const h2v u[9], const Raw& r, f4v* t_lds, int p) {
+  h2v a[6];
+  Cx<float> h[6];
+  project_raw<3, DIR>(r, a);
+  link_mult_h2<DIR>(u, a, h);
+  store_half(t_lds, 0, p, h);
+}
+// (T_LDS: the t hop's half spinor goes to t_lds, at p, for another wave to add)
+template <int W, int DIR, bool T_LDS = false>
+__device__ __forceinline__ void wave_tasks(const f4v* lx, f4v* lh, int p, const WaveLinks& w, Raw& r, Cx<float> acc[12],
+                                           f4v* t_lds = nullptr) {
   constexpr int M0 = W == 3 ? 2 : W == 2 ? 1 : 0, M1 = W == 3 ? 2 : W == 0 ? 0 : 1;
   constexpr bool has_t = DIR > 0 ? W < 3 : W > 0;
   Raw r1, r2;
@@ -107,7 +116,8 @@ __device__ __forceinline__ void wave_tasks(const f4v* lx, f4v* lh, int p, const 
   fence();
   task<M1, DIR>(lh, w, 1, r1);
   fence();
-  if (has_t) t_task<DIR>(w.u[DIR > 0 && W > 0 ? 2 : 3], r2, acc);
+  if (has_t && T_LDS) t_task_lds<DIR>(w.u[DIR > 0 && W > 0 ? 2 : 3], r2, t_lds, p);
+  else if (has_t) t_task<DIR>(w.u[DIR > 0 && W > 0 ? 2 : 3], r2, acc);
   else task<2, DIR>(lh, w, 2, r2);
   fence();
 }
@@ -168,6 +178,58 @@ __device__ __forceinline__ void block_hops(const f4v* lx, f4v* lh, int wave, int
 #undef QWS_WAVE
 }
 
+// The same with the backward hops on four more waves at the same time (helper): their half
+// spinors, those of the t hops with them, in planes of their own, lb.
+__device__ __forceinline__ void block_hops_wide(const f4v* lx, f4v* lh, const f4v* lb, int wave, int p, const WaveLinks& w,
+                                                Cx<float> acc[12]) {
+  Raw r;
+  Halves hs;
+  const Coord l = coord(threadIdx.x, wave);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) acc[k] = {0, 0};
+  __syncthreads();
+#define QWS_WAVE(W)                                \
+  first_raw<W, +1>(lx, w, r);                      \
+  wave_tasks<W, +1>(lx, lh, p, w, r, acc);         \
+  asm volatile("; wave %0" ::"i"(W))
+  if (wave == 0) {
+    QWS_WAVE(0);
+  } else if (wave == 1) {
+    QWS_WAVE(1);
+  } else if (wave == 2) {
+    QWS_WAVE(2);
+  } else {
+    QWS_WAVE(3);
+  }
+#undef QWS_WAVE
+  __syncthreads();
+  sum_halves<+1>(lh, p, l, acc);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) hs.q[3][k] = lb[(9 + k) * VB + p];
+  if (wave > 0) add_half<3, -1>(hs, 2.0f, acc);
+  sum_halves<-1>(lb, p, l, acc);
+}
+__device__ __forceinline__ void helper(const f4v* lx, f4v* lb, int wave, int p, const WaveLinks& w) {
+  Raw r;
+  Cx<float> none[12];
+  __syncthreads();
+#define QWS_WAVE(W)                                             \
+  first_raw<W, -1>(lx, w, r);                                   \
+  wave_tasks<W, -1, true>(lx, lb, p, w, r, none, lb + 9 * VB);  \
+  asm volatile("; wave %0" ::"i"(W))
+  if (wave == 0) {
+    QWS_WAVE(0);
+  } else if (wave == 1) {
+    QWS_WAVE(1);
+  } else if (wave == 2) {
+    QWS_WAVE(2);
+  } else {
+    QWS_WAVE(3);
+  }
+#undef QWS_WAVE
+  __syncthreads();
+}
+
 // y + a x, the multiply-add written out and kept apart from a conversion to FP16 (with
 // which the compiler fuses it in some places only, into one rounding), so that every
 // instantiation rounds alike
@@ -219,24 +281,27 @@ __device__ __forceinline__ void face_produce(const f4v* lx, int j, int p3, int p
 
 // The arguments and steps of k_sap_block_h (sap_kernels.inc), FP16 roundings in the same
 // places; FB: face updates through the face buffer, else by gathers, both with the same
-// roundings.
-template <int NL, bool FB>
-__global__ void __launch_bounds__(VB, 2)
+// roundings.  WIDE: 512 threads, waves 4 to 7 for the backward hops, as in sap4.hip; bit for
+// bit the same.
+template <int NL, bool FB, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 2 * VB : VB, 2)
 k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, const int* __restrict__ active, float kappa,
              int nm, int flags, __half* s, const __half* in, const __half* qface, __half* qout, __half* out,
              const __half* __restrict__ U, const __half* __restrict__ C, float* fb, long long fbs) {
   constexpr int NC = NL / 2;
-  __shared__ f4v sm[12 * VB];
+  __shared__ f4v sm[(WIDE ? 24 : 12) * VB];
   f4v* lh = sm;           // half spinors, float4 [3][3][VB]; in the face update a fourth direction,
   f4v* lx = sm + 9 * VB;  // where the iterate is from then on
+  f4v* lb = sm + 12 * VB;  // WIDE: the backward hops' half spinors, float4 [4][3][VB]
   const unsigned t = threadIdx.x;
   const int j = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wave8 = __builtin_amdgcn_readfirstlane(t >> 6), wave = wave8 & 3;
   const int blk = list[xcd_remap(g, blockIdx.x, gridDim.x)];
   const long long first = (long long)blk * VB, site = first + t;
   h2v cl[36];
 #pragma unroll
   for (int f = 0; f < 18; ++f) {
+    if (WIDE && wave8 >= 4) break;
     typedef _Float16 h4v __attribute__((ext_vector_type(4)));
     const h4v h = __builtin_bit_cast(h4v, ld_nt(reinterpret_cast<const f2v*>(C) + (f * g.V + first) + t));
     cl[2 * f] = h2v{h[0], h[1]}, cl[2 * f + 1] = h2v{h[2], h[3]};
@@ -265,6 +330,19 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
       for (int k = 0; k < 9; ++k) wl.u[i][k] = to_h2(u[i][k]);
     }
   }
+  const int epi = flags & SAP_EPI_MASK;
+  if (WIDE && wave8 >= 4) {  // (the barriers of the other waves' way through the loop below)
+    const int p = lds_pos(t & (VB - 1));
+    for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
+      if (active && !active[r]) continue;
+      __syncthreads();
+      if (FB && (flags & SAP_FACE_PRO)) __syncthreads();
+      for (int it = 0; it < nm; ++it) helper(lx, lb, wave, p, wl);
+      if (epi != SAP_EPI_NONE) helper(lx, lb, wave, p, wl);
+      else __syncthreads();
+    }
+    return;
+  }
   auto face_link = [&](int j, Cx<float> u[9]) {
     const __half* Uo = opaque(U);
     const unsigned s3 = slice_site(wave, 3, j);
@@ -281,13 +359,16 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
   }
   const float tf_hi = b[3] == g.NB[3] - 1 ? 2.0f * g.tbc : 2.0f, tf_lo = b[3] == 0 ? 2.0f * g.tbc : 2.0f;
   const int p = lds_pos(t);
-  const int epi = flags & SAP_EPI_MASK;
 
   for (int r = blockIdx.y; r < nrhs; r += gridDim.y) {
     if (active && !active[r]) continue;  // uniform over the workgroup
     const long long off = r * stride;
     h2v sv[12];
     Cx<float> acc[12];
+    auto hops = [&]() {
+      if (WIDE) block_hops_wide(lx, lh, lb, wave, p, wl, acc);
+      else block_hops(lx, lh, wave, p, wl, acc);
+    };
     load_site(((flags & SAP_SRC_IN) ? in : s) + off, first, g.V, fresh_thread(), sv);
     __syncthreads();  // the previous RHS's readers of lx and lh are done
     if (flags & SAP_FACE_PRO) {
@@ -338,7 +419,7 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
     for (int k = 0; k < 12; ++k) x[k] = sv[k];
     put(lx, p, x);
     for (int it = 0; it < nm; ++it) {
-      block_hops(lx, lh, wave, p, wl, acc);
+      hops();
       fence();
       clover_h2(cl, acc);
 #pragma unroll
@@ -354,7 +435,7 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
 
     if (epi != SAP_EPI_NONE) {
       // acc = T^-1 H_in x
-      block_hops(lx, lh, wave, p, wl, acc);
+      hops();
       const unsigned te = fresh_thread();
       h2v iv[12];
       load_site((epi == SAP_EPI_SUPDATE || (flags & SAP_SRC_IN) ? in : s) + off, first, g.V, epi == SAP_EPI_OUT ? 0 : te, iv);
@@ -407,18 +488,25 @@ k_sap_4444_h(Geo g, const int* __restrict__ list, int nrhs, long long stride, co
 void launch_sap_4444_h(const Geo& g, BlockSel sel, const Batch& B, int nl, float kappa, int nm, int flags, __half* s,
                        const __half* in, const __half* qface, __half* qout, __half* out, const __half* U, const __half* C,
                        float* fb, long long fbs, hipStream_t st) {
-#define SAP4H(NL, FB)                                                                                                  \
-  hipLaunchKernelGGL((k_sap_4444_h<NL, FB>), dim3(sel.n, ny), dim3(VB), 0, st, g, sel.list, B.n, B.stride, B.active, kappa, \
-                     nm, flags, s, in, qface, qout, out, U, C, fb, fbs)
+#define SAP4H(NL, FB, WIDE)                                                                                             \
+  hipLaunchKernelGGL((k_sap_4444_h<NL, FB, WIDE>), dim3(sel.n, ny), dim3(WIDE ? 2 * VB : VB), 0, st, g, sel.list, B.n, \
+                     B.stride, B.active, kappa, nm, flags, s, in, qface, qout, out, U, C, fb, fbs)
+#define SAP4HW(NL, FB)             \
+  do {                             \
+    if (wide) SAP4H(NL, FB, true); \
+    else SAP4H(NL, FB, false);     \
+  } while (0)
   const bool fbk = (flags & (SAP_FACE_OUT | SAP_FACE_FB)) != 0;
   const int ny = sap_rhs_groups(sel.n, B.n, 512);
+  const bool wide = sel.n * ny <= WIDE_GROUPS;
   if (nl == 12) {
-    if (fbk) SAP4H(12, true);
-    else SAP4H(12, false);
+    if (fbk) SAP4HW(12, true);
+    else SAP4HW(12, false);
   } else {
-    if (fbk) SAP4H(18, true);
-    else SAP4H(18, false);
+    if (fbk) SAP4HW(18, true);
+    else SAP4HW(18, false);
   }
+#undef SAP4HW
 #undef SAP4H
 }
 

@@ -59,11 +59,12 @@ def test_msap_h_matches_oracle(prob, nsap, nm):
 
 
 @pytest.mark.parametrize("su3", [True, False])
-@pytest.mark.parametrize("L,nsap,nm", [([8, 8, 8, 8], 2, 1), ([24, 8, 16, 8], 4, 2), ([24, 8, 16, 8], 1, 5)])
+@pytest.mark.parametrize("L,nsap,nm", [([8, 8, 8, 8], 2, 1), ([24, 8, 16, 8], 4, 2), ([24, 8, 16, 8], 1, 5),
+                                       ([24, 8, 16, 16], 3, 2)])
 def test_msap_h_4444(L, nsap, nm, su3):
     """The FP16 kernel for 4^4 blocks (hops by link) where both neighbours of a block are
     the same one, at extents that differ in every direction, with one Jacobi step and
-    several: the oracle's result, by the face buffer bit for bit as by gathers, to the
+    several, by eight waves a block (8 and 48 blocks per colour) and by four (96): the oracle's result, by the face buffer bit for bit as by gathers, to the
     FP16 tolerance of the tests here."""
     p = Problem(L, [4, 4, 4, 4], su3=su3)
     b = p.b.astype(np.float32)
