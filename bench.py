@@ -683,7 +683,7 @@ def main():
             ms_per * 1e-3) / 1e9,
         "roofline": {"bound": "valu", "achieved": achieved_s, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved_s / FP32_PEAK_TFLOPS, "traffic": traffic("sap_f32_32c64_traffic.json"),
-                     "kernel": "k_sap_block<float,12> (fused SAP half-sweep, FP32, %.0f flop/site algorithmic, "
+                     "kernel": "k_sap_4444<12> (fused SAP half-sweep, FP32, %.0f flop/site algorithmic, "
                                "V/2 sites per launch)" % (flops_s / (V / 2)),
                      "ms_per_launch": ms_s,
                      "note": "FP32 vector arithmetic (3x3 complex link products: no MFMA shape); the peak "
