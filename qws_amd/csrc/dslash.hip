@@ -171,7 +171,8 @@ __device__ __forceinline__ void hop_staged(const Geo& g, long long s, const Site
 // algorithmic HBM bytes against 1.48x for k_dslash, 6% faster).  W is the number of
 // waves per SIMD the compiler schedules for (amdgpu_waves_per_eu); at about 104
 // VGPRs 4 waves are resident either way.
-// (Nontemporal link and clover loads were measured slower here, with more L2 misses.)
+// (Nontemporal loads of the links were measured slower, with more L2 misses: the
+// backward hops read them again.)
 template <int NL, int W, bool NT>
 __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_eu(1, W)))
 k_dslash_lds(Geo g, const int* __restrict__ order, int nrhs, long long stride, const int* __restrict__ active, float gamma, float* __restrict__ out,

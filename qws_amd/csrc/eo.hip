@@ -10,7 +10,7 @@
 //   spinor  FP32 float4 [6][Vh], FP64 double2 [12][Vh]
 //   links   [2][4][NL/2][Vh] Vec2  (link from site h of parity p)
 //   clover  [2][18][Vh] float4 / [2][36][Vh] double2
-// One thread per site of the output parity.
+// One thread per site of the output parity, or four on few sites.
 #include <stdexcept>
 #include <type_traits>
 

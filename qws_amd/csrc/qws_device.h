@@ -17,7 +17,8 @@
 //   clover (T^-1): FP32 float4 [18][V] (72 reals), FP64 double2 [36][V],
 //                  FP16 Half4 [18][V]; per site chirality i at reals 36i..36i+35 in
 //                  QWS's packing (clover_def.h:88-284)
-// Every kernel is written for 64-wide wavefronts; one thread owns one site.
+// Every kernel is written for 64-wide wavefronts; a lane owns a site or, in the SAP on
+// 4^4 blocks, a link.
 #pragma once
 
 #include <type_traits>

@@ -7,12 +7,12 @@
 //              (jinv_ddd_in_s_, static_solver.cc:65-140)
 //   epilogue   s_c += in_c - x + kappa T^-1 H_in x,  q_c = x   (qws.cc:814-823)
 //              or the final sequences of prec_ddd_s_ / prec_s_ (qws.cc:842-925, 967-972)
-// The block's forward links and the iterate x live in LDS, the site's clover
-// inverse in registers, so links and clover cross HBM once per half-sweep instead
-// of once per operator application.  Requires proper colouring (face neighbours
-// belong to the other colour) and 256 or 512 sites per block (one thread per site).
-// Instantiated for FP32 storage and for FP16 storage (FP16 operands, FP32
-// accumulation).
+// The kernels here (sap_kernels.inc) hold the block's forward links and the iterate x
+// in LDS, the site's clover inverse in registers, so links and clover cross HBM once
+// per half-sweep instead of once per operator application.  They require proper
+// colouring (face neighbours belong to the other colour) and 256 or 512 sites per
+// block (one thread per site), with FP32 or FP16 storage (FP16 operands, FP32
+// accumulation); 4^4 blocks have kernels of their own (sap4.hip, sap4h.hip).
 #include <type_traits>
 
 #include "kernels.h"
