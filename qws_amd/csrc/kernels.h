@@ -106,9 +106,10 @@ void launch_update_xr(const Batch& B, long long n, R* x, const R* v1, R* r, cons
 // x += alpha v0 (alpha of each RHS)
 template <typename R>
 void launch_update_x(const Batch& B, long long n, R* x, const R* v0, const Scalars* sc, hipStream_t st);
-// p = r + beta (p - omega q)
+// p = r + beta (p - omega q); red |p|^2 if part
 template <typename R>
-void launch_update_p(const Batch& B, long long n, R* p, const R* r, const R* q, const Scalars* sc, hipStream_t st);
+void launch_update_p(const Batch& B, long long n, R* p, const R* r, const R* q, const Scalars* sc, hipStream_t st,
+                     double* part = nullptr);
 template <typename R> void launch_norm(const Batch& B, long long n, const R* a, double* part, hipStream_t st);
 // count: partials per value
 void launch_finalize(const Batch& B, const double* part, int nval, Scalars* sc, int mode, hipStream_t st,

@@ -726,19 +726,22 @@ void Lattice::prec_s_t(const Batch& B, S* out, const S* in, int nsap, int nm) {
 // prec_s_) on an FP16 copy of `in` scaled to unit RMS component; the reference
 // scales to unit norm instead, which leaves large lattices' components in FP16's
 // subnormal range.
-void Lattice::msap_h_t(const Batch& B, float* out, const float* in, int nsap, int nm) {
+void Lattice::msap_h_t(const Batch& B, float* out, const float* in, int nsap, int nm, const Scalars* norm) {
   if (nsap > 10 || nm > 10) throw std::invalid_argument("nsap and nm must be <= 10 (prec_ddd_s_h.h:130-131)");
   ensure_half_fields();
   const int nb = B.n;
   if (!sc_h_) sc_h_ = dalloc<Scalars>(MAX_BATCH);
   __half* ih = (__half*)work("hp_in", spinor_bytes(P16) * nb);
   __half* oh = (__half*)work("hp_out", spinor_bytes(P16) * nb);
-  double* part = reduction_partials(nb);
-  launch_norm<float>(B, g_.V * 12, in, part, st_);
-  launch_finalize(B, part, 1, sc_h_, FIN_RAW, st_);
-  launch_scale_rms<__half, float>(B, g_.V, B.stride, B.stride, ih, in, sc_h_, +1, st_);
+  if (!norm) {
+    double* part = reduction_partials(nb);
+    launch_norm<float>(B, g_.V * 12, in, part, st_);
+    launch_finalize(B, part, 1, sc_h_, FIN_RAW, st_);
+    norm = sc_h_;
+  }
+  launch_scale_rms<__half, float>(B, g_.V, B.stride, B.stride, ih, in, norm, +1, st_);
   prec_s_t<__half>(B, oh, ih, nsap > 1 ? nsap - 1 : 0, nm);
-  launch_scale_rms<float, __half>(B, g_.V, B.stride, B.stride, out, oh, sc_h_, -1, st_);
+  launch_scale_rms<float, __half>(B, g_.V, B.stride, B.stride, out, oh, norm, -1, st_);
 }
 
 void Lattice::msap_h(float* out, const float* in, int nsap, int nm) { msap_h_t(single(), out, in, nsap, nm); }
@@ -1203,7 +1206,8 @@ void Lattice::bicg_t(const Batch& Bin, S* x, const S* b, double tol, int maxiter
   };
   for (int iter = 0; iter < maxiter && any_live(); ++iter) {
     for (int k = 0; k < nb; ++k) iters[k] += live[k];
-    msap_h_t(B, w, p, nsap, nm);
+    // |p|^2 and |r|^2 come with the passes that wrote them (the first p is b)
+    msap_h_t(B, w, p, nsap, nm, iter == 0 ? sc : sc_h_);
     hop<S>(sel(-1), B, HOPS_ALL, mk, q, w, nullptr, nullptr, w);
     launch_dot<S>(B, n, r0, q, part, st_);
     launch_finalize(B, part, 2, sc, FIN_ALPHA, st_);
@@ -1222,14 +1226,15 @@ void Lattice::bicg_t(const Batch& Bin, S* x, const S* b, double tol, int maxiter
       launch_update_x<S>(Batch{nb, B.stride, dfix}, n, x, w, sc, st_);
     }
     if (!more) break;
-    msap_h_t(B, w2, r, nsap, nm);
+    msap_h_t(B, w2, r, nsap, nm, sc);
     hop<S>(sel(-1), B, HOPS_ALL, mk, t, w2, nullptr, nullptr, w2);
     launch_norm_dot<S>(B, n, t, r, part, st_);
     launch_finalize(B, part, 3, sc, FIN_OMEGA, st_);
     launch_update_xr<S>(B, n, x, w2, r, t, sc, 1, r0, part, st_, XR_DEFERRED, w);
     launch_finalize(B, part, 3, sc, FIN_RHO, st_);
     if (!converge()) break;
-    launch_update_p<S>(B, n, p, r, q, sc, st_);  // p = r + beta (p - omega q)
+    launch_update_p<S>(B, n, p, r, q, sc, st_, part);  // p = r + beta (p - omega q)
+    launch_finalize(B, part, 1, sc_h_, FIN_RAW, st_);
   }
   if (trace_on()) {
     read_scalars(sc, nb);

@@ -312,7 +312,8 @@ class Lattice {
   void prec_ddd_t(const Batch& B, S* out, const S* in, int nsap, int nm, const SapSrcUpdate* upd = nullptr);
   template <typename S> void prec_s_t(const Batch& B, S* out, const S* in, int nsap, int nm);
   template <typename S> int bicgstab_dd_t(S* x, const S* b, int maxiter, double tol);
-  void msap_h_t(const Batch& B, float* out, const float* in, int nsap, int nm);
+  // norm: scalars whose red[0] is |in|^2 already, or nullptr
+  void msap_h_t(const Batch& B, float* out, const float* in, int nsap, int nm, const Scalars* norm = nullptr);
   template <typename S>
   void bicg_t(const Batch& B, S* x, const S* b, double tol, int maxiter, int nsap, int nm, std::vector<int>& iters,
               bool hp);

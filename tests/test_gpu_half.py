@@ -131,6 +131,23 @@ def test_inner_hp_solve_true_residual():
     assert np.sqrt(O.norm2(r)) < 3e-5
 
 
+@pytest.mark.parametrize("L,shift", [([8, 8, 8, 8], 40), ([16, 8, 8, 16], -40)])
+def test_inner_hp_solve_scale_invariance(L, shift):
+    """The FP16 copies of p and r take their scale from the sums of the passes that wrote
+    them: a source scaled by a power of two gives the scaled solution bit for bit, in the
+    same number of iterations (every step only moves exponents; a scale off by 2^40 would
+    leave FP16's range)."""
+    p = Problem(L, [4, 4, 4, 4], kappa=0.12, seed=23)
+    b = p.b.astype(np.float32)
+    xs, its = [], []
+    for f in (np.float32(1), np.float32(2.0 ** shift)):
+        x = p.lat.spinor(Q.F32)
+        its.append(p.lat.bicgstab_precdd_h(x, p.lat.spinor(Q.F32, f * b), 1e-6, 100, 3, 2))
+        xs.append(x.download().astype(np.float32) / f)
+    assert its[0] == its[1] and 2 < its[0] < 100
+    assert np.array_equal(xs[0], xs[1])
+
+
 def test_hp_solve_matches_fp32_sap_solve():
     """The FP16-SAP mixed solve reaches the FP64 true residual, and its solution
     agrees with the FP32-SAP solve's (the solution of D x = b is unique)."""
