@@ -108,3 +108,24 @@ def test_driver_helpers(capfd):
     L.get_clock.restype = ctypes.c_double
     t0 = L.get_clock()
     assert t0 > 1.5e9 and L.get_clock() >= t0
+
+
+def test_build_without_the_reference_sources(monkeypatch, tmp_path):
+    """The build leaves the reference library out where the sources are not there, also
+    where their folder exists and is empty."""
+    import subprocess
+
+    import __graft_entry__ as entry
+    from qws_amd import build
+
+    ran = []
+    monkeypatch.setattr(build, "build", lambda jobs: None)
+    monkeypatch.setattr(subprocess, "run", lambda cmd, **k: ran.append(" ".join(cmd)))
+    for refdir in (tmp_path, tmp_path / "none"):
+        monkeypatch.setattr(entry, "REFDIR", str(refdir))
+        entry.build()
+    assert len(ran) == 2 and not any("Makefile.ref" in c for c in ran)
+    (tmp_path / "qws.cc").write_text("")
+    monkeypatch.setattr(entry, "REFDIR", str(tmp_path))
+    entry.build()
+    assert "Makefile.ref" in ran[-1]
