@@ -6,6 +6,7 @@
 // ddd_out_d.cc:84-235 (face hops of a domain, T^-1, out += factor * (...)),
 // qws.cc:625-644 (full operator).  On one GPU the faces are read in place from
 // the neighbouring block instead of being packed and exchanged.
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -308,6 +309,18 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
   }
   if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
     // the full operator (several right-hand sides share their clover through the caches)
+    const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
+    // a grid has fewer than 2^32 work-items: 16 right-hand sides on 32^4 in blocks of one
+    // site, a workgroup each, take two launches
+    const int most = (int)std::max(1LL, ((1LL << 32) - 1) / ((long long)sel.n * wpb * HOP_THREADS));
+    if (B.n > most) {
+      for (int r = 0; r < B.n; r += most) {
+        const Batch part{std::min(most, B.n - r), B.stride, B.active ? B.active + r : nullptr};
+        launch_hop<S, NL>(g, sel, part, set, gamma, out + r * B.stride, in + r * B.stride, nullptr, nullptr,
+                          in + r * B.stride, U, C, st, index_order);
+      }
+      return;
+    }
     Geo gc = g;
     if (index_order && B.n == 1) gc.xcd_chunk = sizeof(S) == 8 ? DSLASH_CHUNK_64 : DSLASH_CHUNK_32;
     const bool nt = B.n == 1 && operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
@@ -333,7 +346,6 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
         return;
       }
     }
-    const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
 #define DSL(NT)                                                                                                  \
   hipLaunchKernelGGL((k_dslash<S, NL, NT>), dim3(sel.n * wpb * B.n), dim3(HOP_THREADS), 0, st, g, sel.list, wpb, B.n, \
                      B.stride, B.active, gamma, out, in, U, C)

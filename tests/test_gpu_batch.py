@@ -63,6 +63,24 @@ def test_right_hand_sides_spread_over_workgroups(L, B, n, sap):
         assert x1.digest() == xs[k].digest(), k
 
 
+def test_batch_of_more_work_items_than_a_launch_takes():
+    """16 right-hand sides on 32^4 in blocks of one site, a workgroup each: 2^32 work-items,
+    one more than a grid may have.  The first and the last two as alone, bit for bit."""
+    lat = Q.Lattice([32, 32, 32, 32], [1, 1, 1, 1], -1, 12, kappa=0.05)
+    lat.generate_gauge(0.3, 13)
+    lat.compute_clover(1.0)
+    n = 16
+    bs = [lat.gaussian(Q.F64, 200 + k) for k in range(n)]
+    xs = [lat.spinor(Q.F64) for _ in range(n)]
+    prm = dict(PRM, nsap=1, nm=1, maxiter=2, maxiter_s=1, true_tol=0, max_restarts=0)
+    lat.solve_batch(xs, bs, **prm)
+    for k in (0, n - 2, n - 1):
+        x1 = lat.spinor(Q.F64)
+        lat.solve(x1, bs[k], **prm)
+        assert x1.digest() == xs[k].digest(), k
+    lat.close()
+
+
 def test_batch_with_initial_guess_and_oracle_residual(lat):
     n = 3
     bs = _sources(lat, n)
