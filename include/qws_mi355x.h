@@ -475,9 +475,11 @@ int qwsg_synchronize(qwsg_lattice* lat);
 int qwsg_time_dslash(qwsg_lattice* lat, int prec, int reps, double* ms_per_call);
 /* Kernel of the FP32 full operator on 256-site blocks: 0 = neighbour gathers from
  * global memory, 3 or 4 = the block's spinor staged in LDS (compiled for 3 or 4
- * waves per SIMD).  The variants give the same results.  qwsg_autotune_dslash
- * times each over `reps` launches on this lattice, keeps the fastest and returns
- * it in *chosen.  Tuning only; no counterpart in the reference. */
+ * waves per SIMD).  Without a call (or QWS_MI355X_DSLASH) it is 4, or on few sites a
+ * kernel with four waves per 64 sites.  All give the same results.
+ * qwsg_autotune_dslash times each over `reps` launches on this lattice and keeps the
+ * fastest; *chosen is 0, 3 or 4, and 4 also where the four-wave kernel is kept.
+ * Tuning only; no counterpart in the reference. */
 int qwsg_set_dslash_kernel(qwsg_lattice* lat, int kernel);
 int qwsg_autotune_dslash(qwsg_lattice* lat, int reps, int* chosen);
 /* Block order of the launches over every block (tuning only): 0 index order, 1 t-z

@@ -487,7 +487,8 @@ class Lattice:
         return ms.value
 
     def set_dslash_kernel(self, k):
-        """FP32 full-operator kernel on 256-site blocks: 0 global gathers, 3/4 LDS-staged."""
+        """FP32 full-operator kernel on 256-site blocks in place of the choice by size:
+        0 global gathers, 3/4 LDS-staged."""
         check(lib().qwsg_set_dslash_kernel(self.h, int(k)))
 
     def autotune_solve(self, x, b, nsaps, nms, **params):

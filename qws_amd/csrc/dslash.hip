@@ -301,13 +301,18 @@ k_dslash_lds_d(Geo g, const int* __restrict__ order, int nrhs, long long stride,
 template <typename S, int NL>
 void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename Store<S>::R gamma, S* out, const S* a,
                 const S* b, const S* c, const S* in, const S* U, const S* C, hipStream_t st, bool index_order) {
-  if (split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value)) {
+  const bool full = set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in;
+  // a kernel that was asked for by name (qwsg_set_dslash_kernel, the environment) is the one that runs
+  const bool named = full && g.Vb == HOP_THREADS &&
+                     ((std::is_same<S, float>::value && g.dslash_kernel != DSLASH_AUTO) ||
+                      (std::is_same<S, double>::value && g.dslash_kernel_d != DSLASH_AUTO));
+  if (!named && split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value)) {
     SplitPart<S> p;
     p.sel = sel, p.set = set, p.gamma = gamma, p.out = out, p.a = a, p.b = b, p.c = c, p.in = in;
     launch_split<S, NL>(g, p, SplitPart<S>(), B, U, C, st);
     return;
   }
-  if (set == HOPS_ALL && sel.n == g.nblk && a == in && b == nullptr && c == nullptr && out != in) {
+  if (full) {
     // the full operator (several right-hand sides share their clover through the caches)
     const int wpb = (g.Vb + HOP_THREADS - 1) / HOP_THREADS;
     // a grid has fewer than 2^32 work-items: 16 right-hand sides on 32^4 in blocks of one
@@ -335,12 +340,12 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
 #define DSL_LDS(W, NT)                                                                                          \
   hipLaunchKernelGGL((k_dslash_lds_d<W, NT>), dim3(sel.n * B.n), dim3(HOP_THREADS), 0, st, gc, sel.list, B.n, B.stride, \
                      B.active, gamma, out, in, U, C)
-        if (g.dslash_kernel_d == 2) {
-          if (nt) DSL_LDS(2, true);
-          else DSL_LDS(2, false);
-        } else {
+        if (g.dslash_kernel_d == 3) {
           if (nt) DSL_LDS(3, true);
           else DSL_LDS(3, false);
+        } else {
+          if (nt) DSL_LDS(2, true);
+          else DSL_LDS(2, false);
         }
 #undef DSL_LDS
         return;

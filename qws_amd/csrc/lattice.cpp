@@ -79,23 +79,23 @@ Lattice::Lattice(const int L[4], const int B[4], int tbc, int links32) {
   // workgroup placement: XCD-contiguous block ranges unless QWS_MI355X_XCD_REMAP=0
   const char* xr = std::getenv("QWS_MI355X_XCD_REMAP");
   g_.xcd_remap = (xr && xr[0] == '0') ? 0 : 1;
-  // full-operator kernel (FP32, 256-site blocks): LDS-staged, compiled for 4 waves per
-  // SIMD, unless QWS_MI355X_DSLASH names another (0, 3, 4); autotune_dslash() times them
+  // full-operator kernel (FP32, 256-site blocks): chosen by size (DSLASH_AUTO) unless
+  // QWS_MI355X_DSLASH names one (0, 3, 4); autotune_dslash() times them
   const char* fbv = std::getenv("QWS_MI355X_SAP_FB");
   use_fb_ = !(fbv && fbv[0] == '0');
   // the inner BiCGStab's direction update inside the first SAP sweep unless QWS_MI355X_SAP_PUPD=0
   const char* pu = std::getenv("QWS_MI355X_SAP_PUPD");
   fold_pupd_ = !(pu && pu[0] == '0');
   const char* dk = std::getenv("QWS_MI355X_DSLASH");
-  g_.dslash_kernel = dk ? std::atoi(dk) : 4;
-  if (g_.dslash_kernel != 0 && g_.dslash_kernel != 3) g_.dslash_kernel = 4;
+  g_.dslash_kernel = dk ? std::atoi(dk) : DSLASH_AUTO;
+  if (g_.dslash_kernel != 0 && g_.dslash_kernel != 3 && g_.dslash_kernel != 4) g_.dslash_kernel = DSLASH_AUTO;
   // FP64 full operator (18-real links, 256-site blocks): LDS-staged for 2 waves per SIMD
   // (32^3x64: 0.82 ms against 0.96-1.02 ms with global gathers, both with contiguous
-  // ranges of blocks for the XCDs; bit-identical), unless
-  // QWS_MI355X_DSLASH_D names another (0 gathers, 3 LDS-staged for 3 waves)
+  // ranges of blocks for the XCDs; bit-identical), or four waves per 64 sites on few
+  // sites, unless QWS_MI355X_DSLASH_D names one (0 gathers, 2 or 3 LDS-staged)
   const char* dkd = std::getenv("QWS_MI355X_DSLASH_D");
-  g_.dslash_kernel_d = dkd ? std::atoi(dkd) : 2;
-  if (g_.dslash_kernel_d != 0 && g_.dslash_kernel_d != 3) g_.dslash_kernel_d = 2;
+  g_.dslash_kernel_d = dkd ? std::atoi(dkd) : DSLASH_AUTO;
+  if (g_.dslash_kernel_d != 0 && g_.dslash_kernel_d != 2 && g_.dslash_kernel_d != 3) g_.dslash_kernel_d = DSLASH_AUTO;
   nl32_ = links32;
   pin_chunk_ = pin_chunk_from_env();
   QWS_HIP(hipStreamCreate(&st_));
@@ -1556,8 +1556,10 @@ int Lattice::autotune_dslash(int reps) {
   if (reps < 1) throw std::invalid_argument("autotune_dslash: reps must be positive");
   int best = g_.dslash_kernel, best_order = dslash_order_;
   double best_ms = 1e30;
+  const bool split = split_pays(g_, HOPS_ALL, g_.nblk * g_.Vb, 1, false);  // else DSLASH_AUTO is 4
   for (int order : {0, 1})
-    for (int k : {0, 3, 4}) {
+    for (int k : {DSLASH_AUTO, 0, 3, 4}) {
+      if (k == DSLASH_AUTO && !split) continue;
       g_.dslash_kernel = k;
       dslash_order_ = order;
       const double ms = time_dslash(P32, reps);
@@ -1569,7 +1571,7 @@ int Lattice::autotune_dslash(int reps) {
     }
   g_.dslash_kernel = best;
   dslash_order_ = best_order;
-  return best;
+  return best == DSLASH_AUTO ? 4 : best;
 }
 
 SolveParams Lattice::autotune_solve(double* x, const double* b, const SolveParams& prm, const std::vector<int>& nsaps,

@@ -209,9 +209,6 @@ class Lattice {
   // average device time (ms) of one fused SAP launch: reps times the 2*nsap + 2
   // launches of one preconditioner application (prec_ddd_s_), single RHS
   double time_sap(int prec, int reps, int nsap, int nm);
-  // FP32 full-operator kernel on 256-site blocks (0 global gathers, 3/4 LDS-staged);
-  // the variants give the same results, autotune_dslash keeps the fastest on this
-  // lattice (timed over `reps` launches each) and returns it
   // FP32 fused SAP: face updates through the face buffer (default) or by gathering
   // the other colour's spinors; both give the same results bit for bit
   void set_sap_face_buffer(bool on) { use_fb_ = on; }
@@ -219,6 +216,10 @@ class Lattice {
   // runs inside the first SAP sweep of the next preconditioner application (default)
   // or as a separate pass; both give the same results bit for bit
   void set_sap_source_update(bool on) { fold_pupd_ = on; }
+  // FP32 full-operator kernel on 256-site blocks (0 global gathers, 3/4 LDS-staged) in
+  // place of the choice by size; all give the same results.  autotune_dslash keeps the
+  // fastest on this lattice (timed over `reps` launches each), the choice by size with
+  // four waves per 64 sites among them, and returns it (4 for the choice by size)
   void set_dslash_kernel(int k);
   // Block order of the launches over every block (the full operator D among them):
   // 0 = index order (x fastest); 1 = inside each XCD's contiguous range of workgroups,
@@ -226,7 +227,6 @@ class Lattice {
   // a block are read while they are still in that XCD's L2.  Results do not depend on it.
   void set_dslash_order(int order);
   int dslash_order() const { return dslash_order_; }
-  int dslash_kernel() const { return g_.dslash_kernel; }
   int autotune_dslash(int reps);
   // The solver's SAP settings tuned on this lattice: one solve of b from x = 0 (x is
   // overwritten) for every (nsap, nm) of the candidate lists with prm's other settings,

@@ -30,6 +30,8 @@
 namespace qws {
 
 // ------------------------------------------------------------------ geometry
+constexpr int DSLASH_AUTO = -1;
+
 struct Geo {
   int L[4];       // lattice extents
   int B[4];       // block extents
@@ -46,8 +48,9 @@ struct Geo {
   int xcd_remap;  // 1: map workgroups to blocks XCD by XCD (xcd_remap), 0: identity
   int xcd_chunk;  // 0: a contiguous range for each XCD, else chunks of so many workgroups in turn
   int dslash_kernel;  // FP32 full operator on 256-site blocks: 0 global gathers (k_dslash),
-                      // 3/4: block spinor staged in LDS, compiled for that many waves per SIMD
-  int dslash_kernel_d;  // the same for FP64 (18-real links): 0 gathers, 2/3 LDS-staged
+                      // 3/4: block spinor staged in LDS, compiled for that many waves per SIMD,
+                      // DSLASH_AUTO: four waves per 64 sites on few sites (split.hip), else as 4
+  int dslash_kernel_d;  // the same for FP64 (18-real links): 0 gathers, 2/3 LDS-staged, DSLASH_AUTO as 2
 };
 
 // MI355X dispatches the workgroups of a launch round-robin over its 8 XCDs, each
