@@ -25,12 +25,17 @@ constexpr int HOP_THREADS = 256;
 constexpr double DSLASH_STREAM_BYTES = 280e6;
 
 // Blocks that an XCD takes in turn in the LDS-staged full operators (xcd_chunk), in index
-// order.  With a contiguous eighth of the lattice for each XCD every face that its L2 has
-// lost comes from memory; side by side the XCDs find it in the last-level cache.  us, a
-// contiguous range / chunks of 8 / of 64:
+// order, above DSLASH_STREAM_BYTES.  With a contiguous eighth of the lattice for each XCD
+// every face that its L2 has lost comes from memory; side by side the XCDs find it in the
+// last-level cache.  us, a contiguous range / chunks of 8 / of 64:
 //   FP64  24^3 48 234 / 214 / 221   32^4 364 / 353 / 348   40 24 32 40 444 / 404 / 412   32^3 64 768 / 681 / 721
 //   FP32  24^3 48  94 /  93 /  93   32^4 152 / 158 / 150   40 24 32 40 187 / 178 / 179   32^3 64 321 / 310 / 313
-// (No gain for k_dslash on large blocks, nor for the even/odd operator.)
+// (No gain for k_dslash on large blocks, nor for the even/odd operator.)  Below that an
+// operator on fields that it has just had finds more of its own range in its L2, and on
+// few blocks the chunks fill the XCDs unevenly.  Three lattices in turn / one again and
+// again, contiguous ranges and chunks:
+//   FP32  16^3 24 11.7 / 19.8 and 14.5 / 21.2   24^4 50.5 / 49.4 and 50.2 / 52.3
+//   FP64  8^2 16 56 16.3 / 22.7 and 16.9 / 23.2   16^3 40 55.7 / 62.0 and 55.3 / 59.7
 constexpr int DSLASH_CHUNK_64 = 8, DSLASH_CHUNK_32 = 64;
 
 template <typename S, int NL, int SET>
@@ -326,9 +331,9 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
       }
       return;
     }
-    Geo gc = g;
-    if (index_order && B.n == 1) gc.xcd_chunk = sizeof(S) == 8 ? DSLASH_CHUNK_64 : DSLASH_CHUNK_32;
     const bool nt = B.n == 1 && operator_bytes<S>(g, NL) > DSLASH_STREAM_BYTES;
+    Geo gc = g;
+    if (index_order && nt) gc.xcd_chunk = sizeof(S) == 8 ? DSLASH_CHUNK_64 : DSLASH_CHUNK_32;
     if constexpr (std::is_same<S, float>::value) {
       if (g.Vb == HOP_THREADS && g.dslash_kernel != 0) {
         launch_dslash_lds<NL>(gc, sel, B, nt, gamma, out, in, U, C, st);
