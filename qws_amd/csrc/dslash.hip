@@ -311,7 +311,7 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
   const bool named = full && g.Vb == HOP_THREADS &&
                      ((std::is_same<S, float>::value && g.dslash_kernel != DSLASH_AUTO) ||
                       (std::is_same<S, double>::value && g.dslash_kernel_d != DSLASH_AUTO));
-  if (!named && split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value)) {
+  if (!named && split_pays(g, set, sel.n * g.Vb, B.n, std::is_same<S, double>::value, NL)) {
     SplitPart<S> p;
     p.sel = sel, p.set = set, p.gamma = gamma, p.out = out, p.a = a, p.b = b, p.c = c, p.in = in;
     launch_split<S, NL>(g, p, SplitPart<S>(), B, U, C, st);

@@ -44,8 +44,10 @@ template <typename S, int NL>
 void launch_split(const Geo& g, const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B, const S* U, const S* C,
                   hipStream_t st);
 
-// Whether launch_split is the faster one for the hop set on that many sites (split.hip).
-bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64);
+// Whether launch_split is the faster one for the hop set on that many sites, or for two
+// operators on that many together (split.hip).
+bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64, int nl);
+bool split_pair_pays(const Geo& g, int sites, int nrhs);
 
 // ---- BiCGStab vector kernels (full lattice, n = number of complex numbers)
 struct Scalars {

@@ -452,8 +452,8 @@ void Lattice::hop(BlockSel s, const Batch& B, int set, typename Store<S>::R gamm
 // Two operators that do not depend on each other: one launch where few sites are at work.
 template <typename S> void Lattice::hop2(const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B) {
   const FieldSet<S> f = fields<S>();
-  // (a pair is worth it to twice the limit of face hops alone: 32 16^3 by halves, FP32 12.6 + 13.6 us and a launch less)
-  if (split_pays(g_, HOPS_FACE, (p0.sel.n + p1.sel.n) * g_.Vb / (p1.sel.n ? 2 : 1), B.n, sizeof(S) == 8)) {
+  if (p1.sel.n ? split_pair_pays(g_, (p0.sel.n + p1.sel.n) * g_.Vb, B.n)
+               : split_pays(g_, p0.set, p0.sel.n * g_.Vb, B.n, sizeof(S) == 8, f.nl)) {
     if (f.nl == 18) launch_split<S, 18>(g_, p0, p1, B, f.U, f.C, st_);
     else if constexpr (!std::is_same<S, double>::value) launch_split<S, 12>(g_, p0, p1, B, f.U, f.C, st_);
     return;
@@ -1556,7 +1556,7 @@ int Lattice::autotune_dslash(int reps) {
   if (reps < 1) throw std::invalid_argument("autotune_dslash: reps must be positive");
   int best = g_.dslash_kernel, best_order = dslash_order_;
   double best_ms = 1e30;
-  const bool split = split_pays(g_, HOPS_ALL, g_.nblk * g_.Vb, 1, false);  // else DSLASH_AUTO is 4
+  const bool split = split_pays(g_, HOPS_ALL, g_.nblk * g_.Vb, 1, false, nl32_);  // else DSLASH_AUTO is 4
   for (int order : {0, 1})
     for (int k : {DSLASH_AUTO, 0, 3, 4}) {
       if (k == DSLASH_AUTO && !split) continue;

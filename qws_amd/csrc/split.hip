@@ -190,32 +190,47 @@ k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2
 
 }  // namespace
 
-// Times in us, k_hop, k_dslash or the staged kernels / this one, on 18-real links:
-//   full operator    8^4 (64 workgroups)  FP32 12.2 / 5.5  FP64 15.3 / 6.4
-//                    16^4, 4^4 blocks (1024)   16.3 / 13.1      24.2 / 23.0
-//                    16^2 32^2, 4^4 blocks (4096) 43.2 / 40.6   98.5 / 98.2
-//                    24^3 32, 4^4 blocks (6912) 78.3 / 80.0    163 / 163: to 4096
-//                    16^3 8, 4^4 blocks (512)   14.5 / 7.7      19.1 / 13.0
-//                    32 12^2 10, halves (720)  11.8 / 10.0      17.0 / 19.3
-//                    48 24^3, halves (10368)   93.2 / 107        285 / 255: FP32 to 4096
-//   inside           48 24^3, halves (5184)    59.4 / 50.6       129 / 117
-//   (32^3 64 by halves is the same either way, by 4^4 blocks up to 8% slower here)
-//   faces            16^4, 4^4 blocks (512)    12.7 / 7.5       16.7 / 12.7
-//                    32 16^3, halves (1024)    11.5 / 12.6      17.6 / 19.7: to 1024
-//   (there most waves of k_hop have no face and leave at once)
-// FP64 has two workgroups per CU (61 KB of LDS): past 512 the second round is nearly
-// empty, and the full operator goes back to k_dslash up to 1024.
-// A block's last workgroup has idle lanes, which blocks under 64 sites pay for with more
-// of them: to 1024 (2^4 blocks, 16384 workgroups: 90 / 100 us).  Right-hand sides share
-// links and clover in k_hop's loop, here only through the caches: to 2048.
-bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64) {
-  if (set == HOPS_NONE || g.Vb >= (1 << 20) || g.V >= (1 << 28)) return false;
-  const long long wg = (long long)(sites / g.Vb) * ((g.Vb + SITES - 1) / SITES) * nrhs;
-  if (set == HOPS_FACE || g.Vb < SITES) return wg <= 1024;
-  if (fp64 && set == HOPS_ALL && wg > 512 && wg < 1024) return false;
-  if (nrhs > 1) return wg <= 2048;
-  return wg <= (set == HOPS_ALL && (g.Vb == 256 || !fp64) ? 4096 : 16384);
+static long long split_groups(const Geo& g, long long sites, int nrhs) {
+  return sites / g.Vb * ((g.Vb + SITES - 1) / SITES) * nrhs;
 }
+static bool split_fits(const Geo& g) { return g.Vb < (1 << 20) && g.V < (1 << 28); }
+
+// The four waves shorten a launch that has the chip for itself; where launches of several
+// streams share it, or one fills it, they are more waves for the same work.  So the limits
+// are where the operator is as fast both ways: us with three lattices on a stream each in
+// turn / with one again and again, first k_hop, k_dslash or the staged kernels, then this
+// one, by workgroups:
+//   full operator, 4^4 blocks  FP32 12-real 512 6.3/13.9 4.4/7.2   1792 13.4/20.6 13.3/18.2   2560 21.8/26.0 24.5/24.1
+//                              18-real 1792 16.3/21.4 16.1/19.6   2560 25.7/28.1 28.1/25.6
+//                              FP64 256 7.6/15.6 4.5/6.9   448 8.8/18.8 7.3/10.7   512 9.5/19.0 9.9/13.8
+//   (times as fast)  x halves  FP32 18-real 720 0.97/1.20, 1024 1.10/0.94, 2560 1.13/1.10, 4000 1.02/1.17
+//                              12-real 720 0.94/1.30, 1024 1.05/1.02, 2592 1.03/1.03, 4000 0.96/1.05
+//                              FP64 720 1.01/0.98, 1024 1.08/0.90, 2048 1.14/1.22, 10368 1.05/1.21
+//   inside, a colour  halves   FP32 18-real 2000 1.05/0.95, 4320 0.97/1.17   12-real 512 1.08/1.3, 1024 0.95/0.97,
+//                              2000 0.95/0.92   FP64 3000 0.98/1.08, 4320 0.96/1.13
+//                    4^4       FP32 512 1.2/1.4, 768 0.87/1.2   FP64 768 1.13/1.02, 3456 1.02/1.13
+//   faces, a colour  halves    FP32 360 1.06/1.37, 512 1.0/1.4, 1024 0.89/0.97   FP64 360 0.99/1.44, 512 0.81/1.25
+//   (there most waves of k_hop have no face and leave at once)
+// FP64 has two workgroups per CU (61 KB of LDS): past 448 a second round begins, nearly
+// empty.  Blocks under 64 sites pay with idle lanes (2^4 blocks, 16384 workgroups: 90 / 100 us
+// alone).  Several right-hand sides share links and clover in k_hop's loop, here only through
+// the caches, but fill the chip better: solves of 3 on 32 12^2 10 by halves (1080 groups a
+// colour) are 1.72 times as fast, with the limits of a single one 1.11 times.
+bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64, int nl) {
+  if (set == HOPS_NONE || !split_fits(g)) return false;
+  const long long wg = split_groups(g, sites, nrhs);
+  const bool all = set == HOPS_ALL, b256 = g.Vb == 256;
+  if (nrhs > 1) return wg <= (set == HOPS_FACE || g.Vb < SITES ? 1024 : 2048) && !(fp64 && all && wg > 512 && wg < 1024);
+  if (wg <= (fp64 ? 448 : 512)) return true;
+  if (set == HOPS_FACE || g.Vb < SITES) return false;
+  if (fp64) return all ? !b256 && wg >= 2048 && wg <= 16384 : wg <= 3072;
+  if (all) return b256 ? wg <= 1792 : wg >= 1024 && wg <= (nl == 12 ? 2592 : 4096);
+  return !b256 && wg <= (nl == 12 ? 768 : 2048);
+}
+// Two operators in one launch, which is worth more: prec_ddd by halves (nsap 4, nm 2), two
+// launches / one, 2048 groups in both: 12-real 1.05/1.05 and 1.02/1.13 times as fast as before
+// there was either, 18-real 1.08/1.09 and 1.05/1.17.
+bool split_pair_pays(const Geo& g, int sites, int nrhs) { return split_fits(g) && split_groups(g, sites, nrhs) <= 2048; }
 
 template <typename S, int NL>
 void launch_split(const Geo& g, const SplitPart<S>& p0, const SplitPart<S>& p1, const Batch& B, const S* U, const S* C,
