@@ -24,7 +24,7 @@ constexpr int HOP_THREADS = 256;
 //   340 MB  77.3 / 69.0    446 MB   108 / 88.9   1409 MB   337 / 313     FP64 1019 MB 253 / 235
 constexpr double DSLASH_STREAM_BYTES = 280e6;
 
-// Blocks that an XCD takes in turn in the LDS-staged full operators (xcd_chunk), in index
+// Blocks that an XCD takes in turn in the LDS-staged full operators (xcd_remap_chunked), in index
 // order, above DSLASH_STREAM_BYTES.  With a contiguous eighth of the lattice for each XCD
 // every face that its L2 has lost comes from memory; side by side the XCDs find it in the
 // last-level cache.  us, a contiguous range / chunks of 8 / of 64:
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(HOP_THREADS) __attribute__((amdgpu_waves_per_e
 k_dslash_lds(Geo g, const int* __restrict__ order, int nrhs, long long stride, const int* __restrict__ active, float gamma, float* __restrict__ out,
              const float* __restrict__ in, const float* __restrict__ U, const float* __restrict__ C) {
   __shared__ float4 lx[6 * HOP_THREADS];
-  int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  int wg = xcd_remap_chunked(g, blockIdx.x, gridDim.x);
   long long off;
   if (!rhs_of(wg, nrhs, stride, active, off)) return;
   in += off, out += off;
@@ -271,7 +271,7 @@ k_dslash_lds_d(Geo g, const int* __restrict__ order, int nrhs, long long stride,
                double* __restrict__ out, const double* __restrict__ in, const double* __restrict__ U,
                const double* __restrict__ C) {
   __shared__ double2 lx[12 * HOP_THREADS];
-  int wg = xcd_remap(g, blockIdx.x, gridDim.x);
+  int wg = xcd_remap_chunked(g, blockIdx.x, gridDim.x);
   long long off;
   if (!rhs_of(wg, nrhs, stride, active, off)) return;
   in += off, out += off;

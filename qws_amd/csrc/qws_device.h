@@ -55,22 +55,22 @@ struct Geo {
 
 // MI355X dispatches the workgroups of a launch round-robin over its 8 XCDs, each
 // with its own L2.  Give XCD x a contiguous range of logical workgroup ids (blocks
-// that share faces then share an L2), or with chunk > 0 every eighth chunk of so many:
-// the XCDs then go through the lattice side by side, and what one fetches another
-// finds in the last-level cache.  A bijection of [0, nwg).
+// that share faces then share an L2).  A bijection of [0, nwg).
 constexpr int NUM_XCD = 8;
-__device__ __forceinline__ int xcd_remap_n(int on, int wg, int nwg, int chunk = 0) {
+__device__ __forceinline__ int xcd_remap_n(int on, int wg, int nwg) {
   if (!on) return wg;
-  const int x = wg % NUM_XCD, i = wg / NUM_XCD;
-  if (chunk > 0) {
-    const int whole = nwg - nwg % (NUM_XCD * chunk);
-    return wg < whole ? (i / chunk * NUM_XCD + x) * chunk + i % chunk : wg;
-  }
   const int q = nwg / NUM_XCD, r = nwg % NUM_XCD;
+  const int x = wg % NUM_XCD, i = wg / NUM_XCD;
   return x * q + (x < r ? x : r) + i;
 }
-__device__ __forceinline__ int xcd_remap(const Geo& g, int wg, int nwg) {
-  return xcd_remap_n(g.xcd_remap, wg, nwg, g.xcd_chunk);
+__device__ __forceinline__ int xcd_remap(const Geo& g, int wg, int nwg) { return xcd_remap_n(g.xcd_remap, wg, nwg); }
+// The same, or with g.xcd_chunk > 0 every eighth chunk of so many: the XCDs then go through
+// the lattice side by side, and what one fetches another finds in the last-level cache.
+__device__ __forceinline__ int xcd_remap_chunked(const Geo& g, int wg, int nwg) {
+  const int chunk = g.xcd_chunk;
+  if (chunk <= 0 || !g.xcd_remap) return xcd_remap(g, wg, nwg);
+  const int x = wg % NUM_XCD, i = wg / NUM_XCD, whole = nwg - nwg % (NUM_XCD * chunk);
+  return wg < whole ? (i / chunk * NUM_XCD + x) * chunk + i % chunk : wg;
 }
 
 // p, hidden from the optimiser.  Loads through the result taken inside a loop over
