@@ -52,7 +52,7 @@ k_hop(Geo g, const int* __restrict__ list, int wg_per_blk, int nrhs, long long s
   const long long s = (long long)blk * g.Vb + loc;
   SiteC sc;
   site_coords(g, s, sc);
-  if (SET == HOPS_FACE && skip_interior) {
+  if ((SET == HOPS_FACE || SET == HOPS_FACE_MASKED) && skip_interior) {
     bool face = false;
 #pragma unroll
     for (int m = 0; m < 4; ++m) face |= (sc.l[m] == 0) | (sc.l[m] == g.B[m] - 1);
@@ -376,7 +376,8 @@ void launch_hop(const Geo& g, BlockSel sel, const Batch& B, int set, typename St
       hipLaunchKernelGGL((k_hop<S, NL, HOPS_INSIDE>), grid, block, 0, st, HOP_ARGS, skip);
       break;
     case HOPS_FACE:
-      hipLaunchKernelGGL((k_hop<S, NL, HOPS_FACE>), grid, block, 0, st, HOP_ARGS, skip);
+      if (g.hopmask == 0xFF) hipLaunchKernelGGL((k_hop<S, NL, HOPS_FACE>), grid, block, 0, st, HOP_ARGS, skip);
+      else hipLaunchKernelGGL((k_hop<S, NL, HOPS_FACE_MASKED>), grid, block, 0, st, HOP_ARGS, skip);
       break;
     default:
       hipLaunchKernelGGL((k_hop<S, NL, HOPS_NONE>), grid, block, 0, st, HOP_ARGS, 0);

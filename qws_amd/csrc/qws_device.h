@@ -42,7 +42,7 @@ struct Geo {
   int nblk;       // number of blocks
   long long V;    // sites
   int tbc;        // +1 periodic / -1 antiperiodic in t
-  int hopmask;    // bit 2*mu + (dir < 0): hop (face hop in HOPS_FACE) taken, 0xFF for all; being a
+  int hopmask;    // bit 2*mu + (dir < 0): hop (face hop in HOPS_FACE_MASKED) taken, 0xFF for all; being a
                   // runtime value it keeps each hop in its own basic block, so the
                   // compiler cannot hoist all eight neighbour loads (256 -> ~146 VGPRs)
   int xcd_remap;  // 1: map workgroups to blocks XCD by XCD (xcd_remap), 0: identity
@@ -454,7 +454,8 @@ __device__ __forceinline__ void clover_apply(const S* C, long long s, long long 
 }
 
 // ------------------------------------------------------------------ hopping sum
-enum HopSet { HOPS_ALL = 0, HOPS_INSIDE = 1, HOPS_FACE = 2, HOPS_NONE = 3 };  // NONE: acc = in (clover only)
+// NONE: acc = in (clover only); FACE_MASKED (of kernels only): the face hops of Geo::hopmask
+enum HopSet { HOPS_ALL = 0, HOPS_INSIDE = 1, HOPS_FACE = 2, HOPS_NONE = 3, HOPS_FACE_MASKED = 4 };
 
 template <int SET>
 __device__ __forceinline__ bool take_hop(bool inside) {
@@ -468,7 +469,7 @@ __device__ __forceinline__ void one_hop(const Geo& g, long long s, const SiteC& 
   bool inside;
   long long n = neighbour(g, s, c, MU, DIR, inside);
   if (!take_hop<SET>(inside)) return;
-  if (SET != HOPS_INSIDE && !(g.hopmask & (1 << (2 * MU + (DIR > 0 ? 0 : 1))))) return;
+  if ((SET == HOPS_ALL || SET == HOPS_FACE_MASKED) && !(g.hopmask & (1 << (2 * MU + (DIR > 0 ? 0 : 1))))) return;
   Cx<R> v[12], a[6], b[6], u[9];
   SpinorIO<S>::load(in, n, g.V, v);
   project<R, MU, DIR>(v, a);
