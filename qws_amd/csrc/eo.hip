@@ -34,7 +34,16 @@ struct EoSite {
   int ick;
 };
 
-__device__ __forceinline__ void eo_coords(const Geo& g, int pe, long long h, EoSite& e) {
+// What the operator takes of Geo: a launch copies its arguments, and the kernel's first
+// loads fetch them from the host (mtilde FP32 12-real with all of Geo / so: 8^4 9.74 / 8.82 us,
+// 16^3 48 32.3 / 31.4).
+struct EoGeo {
+  int L[4];
+  int tbc, xcd_remap;
+  long long V;
+};
+
+template <typename G> __device__ __forceinline__ void eo_coords(const G& g, int pe, long long h, EoSite& e) {
   const int nxh = g.L[0] >> 1;
   long long r = h;
   e.c[0] = (int)(r % nxh); r /= nxh;
@@ -48,7 +57,7 @@ __device__ __forceinline__ void eo_coords(const Geo& g, int pe, long long h, EoS
 // deo_dag_in.cc) into acc; set 1 skips hops that wrap round the lattice ("_in_"),
 // set 2 keeps only those ("_out_pre/_pos"), whose t edge carries 2*tbc.
 template <typename S, int NL, int MU, int DIR, bool DAG, bool NT>
-__device__ __forceinline__ void eo_hop(const Geo& g, int pe, long long h, const EoSite& e, int set, const S* in,
+__device__ __forceinline__ void eo_hop(const EoGeo& g, int pe, long long h, const EoSite& e, int set, const S* in,
                                        const S* U, long long Vh, Cx<typename Store<S>::R> acc[12]) {
   using R = typename Store<S>::R;
   const int nxh = g.L[0] >> 1;
@@ -113,13 +122,13 @@ template <int RED> __device__ __forceinline__ void deo_partials(const double acc
 // mode 0: out = acc, 1: out += fac acc, 2: out = in0 + fac acc.
 template <typename S, int NL, bool DAG, bool NT, int RED>
 __global__ void __launch_bounds__(EO_THREADS)
-k_deo(Geo g, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out, const S* __restrict__ in,
+k_deo(EoGeo g, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out, const S* __restrict__ in,
       const S* in0, const S* __restrict__ U, const S* __restrict__ C, const S* z, double* part) {
   using R = typename Store<S>::R;
   const long long Vh = g.V >> 1;
   // XCD-contiguous ranges of sites: the z and t neighbours a workgroup reads were fetched
   // by workgroups on the same XCD (its L2), not by ones spread round-robin over the XCDs
-  long long h = xcd_remap(g, blockIdx.x, gridDim.x) * (long long)EO_THREADS + threadIdx.x;
+  long long h = xcd_remap_n(g.xcd_remap, blockIdx.x, gridDim.x) * (long long)EO_THREADS + threadIdx.x;
   const bool on = h < Vh;
   if (RED == DEO_STORE && !on) return;
   if (!on) h = Vh - 1;  // (idle, but there for the sums)
@@ -159,7 +168,7 @@ k_deo(Geo g, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* ou
 
 // k_deo (sets 0 to 2) with four waves per 64 sites, for few sites: as k_split of split.hip.
 template <typename S, int NL, int MU, bool DAG, typename Rest>
-__device__ __forceinline__ void eo_two_hops(const Geo& g, int pe, int h, int first, const EoSite& e, bool on, int set,
+__device__ __forceinline__ void eo_two_hops(const EoGeo& g, int pe, int h, int first, const EoSite& e, bool on, int set,
                                             const S* in, const S* U, Cx<typename Store<S>::R> (*lh)[6][split::SITES],
                                             Rest&& rest) {
   using R = typename Store<S>::R;
@@ -221,7 +230,7 @@ __device__ __forceinline__ void eo_two_hops(const Geo& g, int pe, int h, int fir
 
 template <typename S, int NL, bool DAG, int RED>
 __global__ void __launch_bounds__(256, 2)
-k_deo_split(Geo g, float rnx, float ry, float rz, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out,
+k_deo_split(EoGeo g, float rnx, float ry, float rz, int pe, int set, int clv, int mode, typename Store<S>::R fac, S* out,
             const S* __restrict__ in, const S* in0, const S* __restrict__ U, const S* __restrict__ C, const S* z,
             double* part) {
   using R = typename Store<S>::R;
@@ -231,7 +240,7 @@ k_deo_split(Geo g, float rnx, float ry, float rz, int pe, int set, int clv, int 
   __shared__ Cx<R> ly[12][SITES];
   const int lane = threadIdx.x & 63, Vh = (int)(g.V >> 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int first = xcd_remap(g, blockIdx.x, gridDim.x) * SITES;
+  const int first = xcd_remap_n(g.xcd_remap, blockIdx.x, gridDim.x) * SITES;
   const bool on = first + lane < Vh;
   const int h = on ? first + lane : first;
   EoSite e;
@@ -332,14 +341,15 @@ static void deo_launch(const Geo& g, int nl, int pe, int set, int dag, int clv, 
   const bool sp = deo_split_pays(g, set, sizeof(S) == 8);
   if (sp) grid = dim3(deo_split_groups(g));
   const bool nt = (double)g.V * sizeof(S) * (4 * nl + 36 + 24) > DEO_STREAM_BYTES;
+  const EoGeo eg = {{g.L[0], g.L[1], g.L[2], g.L[3]}, g.tbc, g.xcd_remap, g.V};
 #define DEO_ARGS pe, set, clv, mode, fac, out, in, in0, U, C, z, part
 #define DEO(NL, DAG)                                                                                                 \
   do {                                                                                                               \
     if (sp)                                                                                                          \
-      hipLaunchKernelGGL((k_deo_split<S, NL, DAG, RED>), grid, block, 0, st, g, 2.0f / g.L[0], 1.0f / g.L[1],        \
+      hipLaunchKernelGGL((k_deo_split<S, NL, DAG, RED>), grid, block, 0, st, eg, 2.0f / g.L[0], 1.0f / g.L[1],        \
                          1.0f / g.L[2], DEO_ARGS);                                                                   \
-    else if (nt) hipLaunchKernelGGL((k_deo<S, NL, DAG, true, RED>), grid, block, 0, st, g, DEO_ARGS);                \
-    else hipLaunchKernelGGL((k_deo<S, NL, DAG, false, RED>), grid, block, 0, st, g, DEO_ARGS);                       \
+    else if (nt) hipLaunchKernelGGL((k_deo<S, NL, DAG, true, RED>), grid, block, 0, st, eg, DEO_ARGS);                \
+    else hipLaunchKernelGGL((k_deo<S, NL, DAG, false, RED>), grid, block, 0, st, eg, DEO_ARGS);                       \
   } while (0)
   if constexpr (RED != DEO_STORE) {
     if (nl != 18 || dag || set != 0 || mode != 2) throw std::logic_error("deo_launch: sums with the FP64 operator only");

@@ -686,7 +686,6 @@ void Lattice::prec_ddd_t(const Batch& B, S* out, const S* in, int nsap, int nm, 
 // prec_s_ (qws.cc:929-975): out = M_SAP in
 template <typename S>
 void Lattice::prec_s_t(const Batch& B, S* out, const S* in, int nsap, int nm) {
-  using R = typename Store<S>::R;
   const int pr = sizeof(S) == 8 ? P64 : sizeof(S) == 4 ? P32 : P16;
   S* s = (S*)work("sap_s", spinor_bytes(pr) * B.n);
   S* q = (S*)work("sap_q", spinor_bytes(pr) * B.n);

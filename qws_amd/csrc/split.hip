@@ -18,10 +18,29 @@ using namespace split;
 
 namespace {
 
+// What the kernel takes of Geo, and all its arguments in one, with a second operator only
+// where there is one: a launch copies them, and the kernel's first loads fetch them from
+// the host (Geo and two operators each time / so: D on 8^4, FP32, 3.44 / 3.34 us a call with
+// three lattices in turn, 5.31 / 5.24 with one).
+struct SplitGeo {
+  int B[4], NB[4], sB[4], sN[4];
+  int Vb, tbc, hopmask, xcd_remap;
+  long long V;
+};
+template <typename S, bool PAIR> struct SplitArgs {
+  SplitGeo g;
+  float rb[3];
+  int wg_per_blk;
+  long long stride;
+  const int* active;
+  const S *U, *C;
+  SplitPart<S> p[PAIR ? 2 : 1];
+};
+
 // The two hops of wave MU: half spinors into lh, zero for a hop that is not taken.
 // rest() loads the clover.  FP64: a hop at a time, there are no registers for both.
 template <typename S, int NL, int MU, typename Rest>
-__device__ __forceinline__ void two_hops(const Geo& g, int s, int first, const int b[4], const int l[4], bool on, int set,
+__device__ __forceinline__ void two_hops(const SplitGeo& g, int s, int first, const int b[4], const int l[4], bool on, int set,
                                          int mask, const S* in, const S* U,
                                          Cx<typename Store<S>::R> (*lh)[6][SITES], Rest&& rest) {
   using R = typename Store<S>::R;
@@ -80,19 +99,19 @@ __device__ __forceinline__ void two_hops(const Geo& g, int s, int first, const i
   asm volatile("; end of direction %0" ::"i"(MU));
 }
 
-template <typename S, int NL>
-__global__ void __launch_bounds__(256)
-k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2, int wg_per_blk, long long stride,
-        const int* __restrict__ active, const S* __restrict__ U, const S* __restrict__ C) {
+template <typename S, int NL, bool PAIR>
+__global__ void __launch_bounds__(256) k_split(SplitArgs<S, PAIR> args) {
   using R = typename Store<S>::R;
   __shared__ Cx<R> lh[8][6][SITES];
   __shared__ Cx<R> ly[12][SITES];
-  if (active && !active[blockIdx.y]) return;
+  const SplitGeo& g = args.g;
+  if (args.active && !args.active[blockIdx.y]) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = p0.sel.n * wg_per_blk;
-  const bool second = (int)blockIdx.x >= n0;
-  const int wg = second ? xcd_remap(g, blockIdx.x - n0, gridDim.x - n0) : xcd_remap(g, blockIdx.x, n0);
+  const SplitPart<S>&p0 = args.p[0], &p1 = args.p[PAIR ? 1 : 0];
+  const int wg_per_blk = args.wg_per_blk, n0 = PAIR ? p0.sel.n * wg_per_blk : (int)gridDim.x;
+  const bool second = PAIR && (int)blockIdx.x >= n0;
+  const int wg = second ? xcd_remap_n(g.xcd_remap, blockIdx.x - n0, gridDim.x - n0) : xcd_remap_n(g.xcd_remap, blockIdx.x, n0);
   const int* list = second ? p1.sel.list : p0.sel.list;
   const int set = second ? p1.set : p0.set, mask = g.hopmask & (second ? p1.mask : p0.mask);
   const R gamma = second ? p1.gamma : p0.gamma;
@@ -101,6 +120,8 @@ k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2
   const S* tb = second ? p1.b : p0.b;
   const S* tc = second ? p1.c : p0.c;
   const S* in = second ? p1.in : p0.in;
+  const S* __restrict__ U = args.U;
+  const S* __restrict__ C = args.C;
   const int bi = wg / wg_per_blk, blk = list ? list[bi] : bi;
   const int loc0 = (wg - bi * wg_per_blk) * SITES;
   const int loc = loc0 + lane < g.Vb ? loc0 + lane : loc0;
@@ -115,7 +136,7 @@ k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2
   b[3] = rem;
   // loc / B by the reciprocal: exact below 2^20
   {
-    const int q0 = (int)((loc + 0.5f) * rb0), q1 = (int)((q0 + 0.5f) * rb1), q2 = (int)((q1 + 0.5f) * rb2);
+    const int q0 = (int)((loc + 0.5f) * args.rb[0]), q1 = (int)((q0 + 0.5f) * args.rb[1]), q2 = (int)((q1 + 0.5f) * args.rb[2]);
     l[0] = loc - q0 * g.B[0], l[1] = q0 - q1 * g.B[1], l[2] = q1 - q2 * g.B[2], l[3] = q2;
   }
   if (set == HOPS_FACE && out == ta && !tb && !tc) {  // sites without a face hop keep out
@@ -128,7 +149,7 @@ k_split(Geo g, SplitPart<S> p0, SplitPart<S> p1, float rb0, float rb1, float rb2
   const R tf_hi = b[3] == g.NB[3] - 1 && l[3] == g.B[3] - 1 ? R(2 * g.tbc) : R(2);
   const R tf_lo = b[3] == 0 && l[3] == 0 ? R(2 * g.tbc) : R(2);
 
-  const long long off = blockIdx.y * stride;
+  const long long off = blockIdx.y * args.stride;
   R ca[36];  // chirality wave & 1 of T^-1
   auto rest = [&]() { IO<S>::chir(C, wave & 1, g.V, sa * IO<S>::Q, ca); };
   const S* src = in + off;
@@ -239,8 +260,18 @@ void launch_split(const Geo& g, const SplitPart<S>& p0, const SplitPart<S>& p1, 
   const int wpb = (g.Vb + SITES - 1) / SITES;
   const int n = (p0.sel.n + p1.sel.n) * wpb;
   if (n == 0) return;
-  hipLaunchKernelGGL((k_split<S, NL>), dim3(n, B.n), dim3(256), 0, st, g, p0, p1, 1.0f / g.B[0], 1.0f / g.B[1], 1.0f / g.B[2],
-                     wpb, B.stride, B.active, U, C);
+  SplitArgs<S, true> args;
+  for (int m = 0; m < 4; ++m) args.g.B[m] = g.B[m], args.g.NB[m] = g.NB[m], args.g.sB[m] = g.sB[m], args.g.sN[m] = g.sN[m];
+  args.g.Vb = g.Vb, args.g.tbc = g.tbc, args.g.hopmask = g.hopmask, args.g.xcd_remap = g.xcd_remap, args.g.V = g.V;
+  for (int m = 0; m < 3; ++m) args.rb[m] = 1.0f / g.B[m];
+  args.wg_per_blk = wpb, args.stride = B.stride, args.active = B.active, args.U = U, args.C = C;
+  args.p[0] = p0, args.p[1] = p1;
+  if (p1.sel.n) {
+    hipLaunchKernelGGL((k_split<S, NL, true>), dim3(n, B.n), dim3(256), 0, st, args);
+  } else {
+    const SplitArgs<S, false> one = {args.g, {args.rb[0], args.rb[1], args.rb[2]}, wpb, B.stride, B.active, U, C, {p0}};
+    hipLaunchKernelGGL((k_split<S, NL, false>), dim3(n, B.n), dim3(256), 0, st, one);
+  }
 }
 
 #define INST_SPLIT(S, NL)                                                                                            \
