@@ -319,18 +319,21 @@ k_deo_split(EoGeo g, float rnx, float ry, float rz, int pe, int set, int clv, in
   if (RED != DEO_STORE) deo_partials<RED>(red, part);
 }
 
-// Whether k_deo_split is the faster one: by its workgroups (64 sites).  mtilde in us with
-// k_deo / with it, 18-real links:
-//   workgroups   32          256         512         768         1024        1536        2048        3456
-//   FP32         16.8 / 9.8  17.4 / 10.5 23.4 / 14.7 25.8 / 20.4 28.4 / 26.5 35.2 / 36.0 44.0 / 46.8 94.4 / 76.1
-//   FP64         19.8 / 11.3 25.7 / 14.9 30.4 / 27.1 36.2 / 37.9 52.2 / 50.1 84 / 70     100 / 100   181 / 201
-// FP32 also wins from three full rounds on (768 workgroups each; 2304: 53.6 / 50.7) to 4096
-// (5184: 145 / 151); FP64's gains past 512 come and go with its rounds of 512.
+// Whether k_deo_split is the faster one: by its workgroups (64 sites), where it is no slower
+// with three lattices on a stream each in turn / with one again and again.  mtilde in us, k_deo,
+// then it:
+//   workgroups      32                 256               1024                1280
+//   FP32 12-real    7.9/16.6 7.8/8.8   8.6/17.1 7.9/9.3  18.2/26.1 17.1/24.0 22.6/29.6 21.1/27.7
+//        18-real    7.7/16.5 6.3/10.0  9.2/17.8 6.3/10.4 20.8/28.1 20.3/27.3 27.8/32.0 26.1/31.8
+//   workgroups      128                256               512
+//   FP64            11.0/20.2 8.4/11.9 13.6/25.3 10.5/15.1 22.8/30.1 21.5/26.2
+// Past that the chip is full and its waves only more: FP32 2304 to 4096 workgroups 0.94 to 0.98
+// times as fast with three lattices (alone 0.95 to 1.21), FP64 768 36.2 / 37.9 alone.
 static int deo_split_groups(const Geo& g) { return (int)(((g.V >> 1) + split::SITES - 1) / split::SITES); }
 static bool deo_split_pays(const Geo& g, int set, bool fp64) {
   const int n = deo_split_groups(g);
   if (set == 3 || (g.V >> 1) >= (1 << 20)) return false;
-  return fp64 ? n <= 512 : n <= 1280 || (n >= 2304 && n <= 4096);
+  return n <= (fp64 ? 512 : 1280);
 }
 
 template <typename S, int RED>
