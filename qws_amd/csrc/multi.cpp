@@ -182,7 +182,7 @@ void Fused::prec(std::vector<PrecJob>& jobs, bool ddd, int nsap, int nm, SapFusi
     m.b4 = sap_is_4444(L0.g_);
     int most = 1;
     for (const PrecJob& j : jobs) most = std::max(most, j.B.n);
-    m.rhs = sap_rhs_groups(m.n, most, s0.face ? 1024 : vb == 256 ? 512 : 256);
+    m.rhs = sap_rhs_groups(m.n, most, s0.face ? 1024 : sap_slots(vb, nl, true, m.b4 != 0));
     Rec r;
     std::memset(&r, 0, sizeof(r));
     r.m = m, r.flags = s0.flags | (s0.pupd ? SAP_SRC_PUPD : 0), r.face = s0.face ? 1 : 0;

@@ -76,6 +76,11 @@ inline int sap_rhs_groups(int blocks, int nrhs, int slots) {
   return best;
 }
 
+// Workgroups of a half-sweep launch that run at once: two per CU where the LDS holds two
+// (18-real FP32 links of 256 sites take 98 KB in the general kernel: solves of 3 right-hand
+// sides on 16^3 x 32 in 8x4x4x2 blocks with 512 / 256 here 21.3 / 19.9 ms, of 12 70.5 / 69.2).
+inline int sap_slots(int vb, int nl, bool fp32, bool b4) { return vb == 256 && (b4 || !fp32 || nl == 12) ? 512 : 256; }
+
 bool sap_fusable(const Geo& g);
 // 4^4 blocks: the kernels of sap4.hip and sap4h.hip
 bool sap_is_4444(const Geo& g);

@@ -29,7 +29,7 @@ static void check_face_flags(int flags) {
 }
 
 namespace sap256 {
-constexpr int VB = 256;  // 4^4 blocks
+constexpr int VB = 256;
 #include "sap_kernels.inc"
 }  // namespace sap256
 namespace sap512 {
