@@ -213,6 +213,36 @@ def test_eo_bicgstab_stops_at_either_half_step(L):
     assert len(its) > 4
 
 
+@pytest.mark.parametrize("L", [[8, 4, 4, 8], [12, 16, 12, 32], [24, 24, 24, 20]])
+def test_eo_bicgstab_where_the_next_operator_waits(L):
+    """Solves that start near their solution, or end soon after: done in the first half-step
+    or in one within a factor of 10 of tol, whose next operator waits for the check, x being
+    updated at once or (above 2^18 sites) at the end.  The largest lattice's operator (292 MB)
+    goes past the caches, its sums with it.  True residual as above."""
+    lat = Q.Lattice(L, [L[0] // 2] + L[1:], -1, 18, kappa=0.115)
+    lat.generate_gauge(0.3, 4)
+    lat.compute_clover(1.0)
+    lat.eo_from_lattice()
+    bh = np.random.default_rng(3).standard_normal((lat.V // 2, 24))
+    b, q = lat.eo_spinor(Q.F64, bh), lat.eo_spinor(Q.F64)
+    for start, tols in ((1e-6, (1e-5, 1e-6, 7e-7, 4e-7, 1e-7)), (1, (0.5, 0.1, 0.03, 0.01, 1e-8))):
+        x0 = np.zeros_like(bh)
+        if start < 1:
+            x = lat.eo_spinor(Q.F64, x0)
+            lat.eo_bicgstab(x, b, maxiter=200, tol=start)
+            x0 = x.download()
+        its = []
+        for tol in tols:
+            x = lat.eo_spinor(Q.F64, x0)
+            its.append(lat.eo_bicgstab(x, b, maxiter=200, tol=tol))
+            lat.mtilde(q, x, 0, 0)
+            assert rel(q.download(), bh) < tol * (1 + 1e-6) + 1e-10
+        assert its[0] == 1 and its[-1] > 1, its
+        x = lat.eo_spinor(Q.F64, x0)
+        assert lat.eo_bicgstab(x, b, maxiter=1, tol=0.5) == 1  # no iteration: x as it was
+        assert np.array_equal(x.download(), x0)
+
+
 def test_mtilde_is_schur_complement_of_d():
     """Even extents, fields gathered from the lattice's own: with y_e = x and
     y_o = kappa T_oo^-1 H_oe x, the full D gives (D y)_o = 0 and (D y)_e = mtilde x
