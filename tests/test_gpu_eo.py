@@ -243,6 +243,29 @@ def test_eo_bicgstab_where_the_next_operator_waits(L):
         assert np.array_equal(x.download(), x0)
 
 
+@pytest.mark.parametrize("L,links", [([24, 24, 24, 28], 18), ([24, 24, 24, 34], 12)])
+def test_deo_beyond_the_caches(L, links):
+    """Operators of more than 200 MB, whose links and clover are read and whose results are
+    written past the caches (FP32 204 and 203 MB, FP64 409 and 496): with in0 = y on one
+    parity, in = y on the other and fac = -kappa, the full operator D y on that parity."""
+    lat = Q.Lattice(L, [L[0] // 2] + L[1:], -1, links, kappa=0.11)
+    lat.generate_gauge(0.3, 6)
+    lat.compute_clover(1.0)
+    lat.eo_from_lattice()
+    orc = O.Oracle(L, [L[0] // 2] + L[1:], -1, 0.11, lat.gauge(), lat.clover_field())
+    y = np.random.default_rng(29).standard_normal((lat.V, 24))
+    t, z, yy, xh = np.indices((L[3], L[2], L[1], L[0] // 2)).reshape(4, -1)
+    site = lambda p: 2 * xh + (p + yy + z + t) % 2 + L[0] * (yy + L[1] * (z + L[2] * t))
+    for prec, dt, tol in ((Q.F64, np.float64, 1e-13), (Q.F32, np.float32, 1e-6)):
+        d = orc.dslash(y.astype(dt).reshape(-1, 3, 4, 2)).reshape(-1, 24)
+        for pe in (0, 1):
+            out = lat.eo_spinor(prec)
+            lat.deo(out, lat.eo_spinor(prec, y[site(1 - pe)]), pe, clv=True, mode=2, fac=-0.11,
+                    in0=lat.eo_spinor(prec, y[site(pe)]))
+            assert rel(out.download(), d[site(pe)]) < tol, (pe, prec)
+    lat.close()
+
+
 def test_mtilde_is_schur_complement_of_d():
     """Even extents, fields gathered from the lattice's own: with y_e = x and
     y_o = kappa T_oo^-1 H_oe x, the full D gives (D y)_o = 0 and (D y)_e = mtilde x
