@@ -688,6 +688,51 @@ def test_fp64_dslash_kernels_agree_bitwise(monkeypatch):
     assert digests[0] == digests[1] == digests[2]
 
 
+@pytest.mark.parametrize("links", [12, 18])
+def test_full_operators_beyond_the_last_level_cache(monkeypatch, links):
+    """24^3 x 32 in 4^4 blocks, 297 MB and more in FP32 and 679 MB in FP64: clover and results
+    past the caches, blocks in chunks over the XCDs in index order and in contiguous ranges in
+    pencil order.  Every kernel gives the gathering one's result bit for bit, the oracle's to
+    rounding; so does D by halves of 3456 groups of 64 sites (FP64 by four waves per group)."""
+    L = [24, 24, 24, 32]
+    lat = Q.Lattice(L, [4, 4, 4, 4], -1, links, kappa=0.12)
+    lat.generate_gauge(0.3, 7)
+    lat.compute_clover(1.0)
+    U, C = lat.gauge(), lat.clover_field()
+    orc = O.Oracle(L, [4, 4, 4, 4], -1, 0.12, U, C)
+    b = np.random.default_rng(31).standard_normal((lat.V, 3, 4, 2))
+    for prec, dt, tol in ((Q.F32, np.float32, TOL32), (Q.F64, np.float64, TOL64)):
+        want = orc.dslash(b.astype(dt))
+        digests = set()
+        for kd in (("0", "2", "3") if prec == Q.F64 else ("2",)):
+            monkeypatch.setenv("QWS_MI355X_DSLASH_D", kd)
+            one = Q.Lattice(L, [4, 4, 4, 4], -1, links, kappa=0.12)
+            one.load_gauge(U)
+            one.load_clover(C)
+            inp, o = one.spinor(prec, b.astype(dt)), one.spinor(prec)
+            for order in (0, 1):
+                one.set_dslash_order(order)
+                for k in ((0, 3, 4) if prec == Q.F32 else (None,)):
+                    if k is not None:
+                        one.set_dslash_kernel(k)
+                    o.zero()
+                    one.dslash(o, inp)
+                    digests.add(o.digest())
+            one.close()
+        o = lat.spinor(prec)
+        lat.dslash(o, lat.spinor(prec, b.astype(dt)))
+        assert digests == {o.digest()}, prec
+        assert rel(o.download(), want) < tol
+    lat.close()
+    lat = Q.Lattice(L, [12, 24, 24, 32], -1, links, kappa=0.12)
+    lat.load_gauge(U)
+    lat.load_clover(C)
+    o = lat.spinor(Q.F64)
+    lat.dslash(o, lat.spinor(Q.F64, b))
+    assert rel(o.download(), want) < TOL64
+    lat.close()
+
+
 def test_links12_reconstruction():
     """12-real FP32 links (third row rebuilt) equal 18-real storage for SU(3) links."""
     p = Problem([8, 8, 4, 8], [4, 4, 2, 4], su3=True, seed=11)
