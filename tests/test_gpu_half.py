@@ -97,6 +97,22 @@ def test_msap_h_face_buffer_is_bitwise_the_gather(L, B, su3):
     assert rel(res[True], p.orc.msap_h(b, 3, 2)) < 2 * TOL_H
 
 
+@pytest.mark.parametrize("B,su3", [([8, 4, 4, 2], True), ([8, 4, 4, 2], False), ([4, 4, 2, 8], True)])
+def test_msap_h_on_other_256_site_blocks(B, su3):
+    """The general FP16 kernel on blocks of 256 sites that are not 4^4: face buffer and gathers
+    bit for bit alike, and the oracle's result to the FP16 tolerance."""
+    p = Problem([16, 8, 8, 16], B, su3=su3)
+    b = p.b.astype(np.float32)
+    res = []
+    for fb in (True, False):
+        p.lat.set_sap_face_buffer(fb)
+        out = p.lat.spinor(Q.F32)
+        p.lat.msap_h(out, p.lat.spinor(Q.F32, b), 3, 2)
+        res.append(out.download())
+    assert np.array_equal(*res)
+    assert rel(res[0], p.orc.msap_h(b, 3, 2)) < 2 * TOL_H
+
+
 def test_msap_h_links12():
     """12-real links: the third row is rebuilt in FP32 from the FP16 rows 0 and 1,
     so the oracle (which rounds all 18 reals) agrees to a few FP16 roundings."""

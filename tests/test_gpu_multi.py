@@ -56,6 +56,27 @@ def test_fused_multi_lattice_solve_is_each_lattice_alone(shapes):
         lat.close()
 
 
+@pytest.mark.parametrize("B,links", [([8, 4, 4, 2], 12), ([8, 4, 4, 2], 18), ([8, 4, 4, 4], 12)])
+def test_fused_multi_lattice_solve_on_other_blocks(B, links):
+    """The general half-sweep kernel over several lattices, with several right-hand sides a
+    block: each lattice's own result bit for bit."""
+    parts = []
+    for i, (L, n) in enumerate((([16, 8, 8, 8], 4), ([16, 8, 8, 16], 1), ([16, 16, 8, 8], 3))):
+        lat = Q.Lattice(L, B, -1, links, kappa=0.128)
+        lat.generate_gauge(0.3, 40 + i)
+        lat.compute_clover(1.0)
+        parts.append((lat, [lat.spinor(Q.F64) for _ in range(n)], [lat.gaussian(Q.F64, 10 * i + k) for k in range(n)]))
+    prm = dict(SOLVE, nm=3)
+    fused = Q.solve_multi(parts, **prm)
+    for (lat, xs, bs), st in zip(parts, fused):
+        alone_x = [lat.spinor(Q.F64) for _ in xs]
+        alone = lat.solve_batch(alone_x, bs, **prm)
+        for k in range(len(xs)):
+            assert alone_x[k].digest() == xs[k].digest(), (lat.L, k)
+            assert st[k]["inner_iters"] == alone[k]["inner_iters"] and st[k]["true_residual"] <= 1e-10
+        lat.close()
+
+
 def test_fused_multi_lattice_solve_rejects_bad_input():
     a = _lattice([8, 8, 8, 8], 0.12, 0.3, 3)
     x, b = a.spinor(Q.F64), a.gaussian(Q.F64, 1)

@@ -733,6 +733,25 @@ def test_full_operators_beyond_the_last_level_cache(monkeypatch, links):
     lat.close()
 
 
+@pytest.mark.parametrize("B,su3", [([8, 4, 4, 2], True), ([8, 4, 4, 2], False), ([4, 4, 2, 8], True)])
+def test_fused_sap_on_other_256_site_blocks(B, su3):
+    """The general half-sweep kernel on blocks of 256 sites that are not 4^4, with 12-real and
+    18-real links: face buffer and gathers bit for bit alike, and the oracle's result."""
+    p = Problem([16, 8, 8, 16], B, kappa=0.125, seed=9, su3=su3)
+    src = p.b.astype(np.float32)
+    res = []
+    for fb in (True, False):
+        p.lat.set_sap_face_buffer(fb)
+        o1, o2 = p.lat.spinor(Q.F32), p.lat.spinor(Q.F32)
+        p.lat.prec_ddd(o1, p.lat.spinor(Q.F32, src), 2, 3)
+        p.lat.prec_s(o2, p.lat.spinor(Q.F32, src), 2, 3)
+        res.append((o1.download(), o2.download()))
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
+    assert rel(res[0][0], p.orc.prec_ddd_s(src, 2, 3)) < 5e-6
+    assert rel(res[0][1], p.orc.prec_s(src, 2, 3)) < 5e-6
+
+
 def test_links12_reconstruction():
     """12-real FP32 links (third row rebuilt) equal 18-real storage for SU(3) links."""
     p = Problem([8, 8, 4, 8], [4, 4, 2, 4], su3=True, seed=11)
