@@ -147,6 +147,18 @@ def test_inner_hp_solve_true_residual():
     assert np.sqrt(O.norm2(r)) < 3e-5
 
 
+@pytest.mark.parametrize("L", [[8, 8, 8, 8], [16, 8, 8, 16]])
+def test_inner_hp_solve_scales_p_and_r_by_their_own_norms(L):
+    """D near 1, where M is D^-1 but for FP16's roundings: a half-step takes the residual down
+    by their size, 4e-4, four to 2e-14 and six to 1e-20.  A copy of p or r scaled by any other
+    vector's norm (the source's, the p of the last iteration) lies 1e-4 to 1e-7 below 1, in
+    FP16's subnormal range, and its half-step gains at most 0.1: 1e-11 and 1e-16."""
+    p = Problem(L, [4, 4, 4, 4], kappa=0.005, seed=27)
+    for tol, its in ((1e-12, 2), (1e-18, 3)):
+        x = p.lat.spinor(Q.F32)
+        assert p.lat.bicgstab_precdd_h(x, p.lat.spinor(Q.F32, p.b.astype(np.float32)), tol, 20, 3, 2) == its
+
+
 @pytest.mark.parametrize("L,shift", [([8, 8, 8, 8], 40), ([16, 8, 8, 16], -40)])
 def test_inner_hp_solve_scale_invariance(L, shift):
     """The FP16 copies of p and r take their scale from the sums of the passes that wrote
