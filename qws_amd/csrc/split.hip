@@ -217,16 +217,16 @@ static long long split_groups(const Geo& g, long long sites, int nrhs) {
 static bool split_fits(const Geo& g) { return g.Vb < (1 << 20) && g.V < (1 << 28); }
 
 // The four waves shorten a launch that has the chip for itself; where launches of several
-// streams share it, or one fills it, they are more waves for the same work.  So the limits
-// are where the operator is as fast both ways: us with three lattices on a stream each in
-// turn / with one again and again, first k_hop, k_dslash or the staged kernels, then this
-// one, by workgroups:
+// streams share it, or one fills it, they are more waves for the same work.  So this kernel
+// has the sizes at which it is no slower with three lattices on a stream each in turn, if one
+// again and again, its fields in the caches, does not lose as much: us in turn / again and
+// again, first k_hop, k_dslash or the staged kernels, then this one, by workgroups:
 //   full operator, 4^4 blocks  FP32 12-real 512 6.3/13.9 4.4/7.2   1792 13.4/20.6 13.3/18.2   2560 21.8/26.0 24.5/24.1
 //                              18-real 1792 16.3/21.4 16.1/19.6   2560 25.7/28.1 28.1/25.6
 //                              FP64 256 7.6/15.6 4.5/6.9   448 8.8/18.8 7.3/10.7   512 9.5/19.0 9.9/13.8
-//   (times as fast)  x halves  FP32 18-real 720 0.97/1.20, 1024 1.10/0.94, 2560 1.13/1.10, 4000 1.02/1.17
+//   (times as fast)  x halves  FP32 18-real 720 0.97/1.20, 1024 1.13/0.92, 1664 1.22/0.88, 2560 1.13/1.10, 4000 1.02/1.17
 //                              12-real 720 0.94/1.30, 1024 1.05/1.02, 2592 1.03/1.03, 4000 0.96/1.05
-//                              FP64 720 1.01/0.98, 1024 1.08/0.90, 2048 1.14/1.22, 10368 1.05/1.21
+//                              FP64 720 1.01/0.98, 1024 1.12/0.95, 1152 1.20/1.06, 2048 1.13/1.22, 10368 1.05/1.21
 //   inside, a colour  halves   FP32 18-real 2000 1.05/0.95, 4320 0.97/1.17   12-real 512 1.08/1.3, 1024 0.95/0.97,
 //                              2000 0.95/0.92   FP64 3000 0.98/1.08, 4320 0.96/1.13
 //                    4^4       FP32 512 1.2/1.4, 768 0.87/1.2   FP64 768 1.13/1.02, 3456 1.02/1.13
@@ -244,7 +244,7 @@ bool split_pays(const Geo& g, int set, int sites, int nrhs, bool fp64, int nl) {
   if (nrhs > 1) return wg <= (set == HOPS_FACE || g.Vb < SITES ? 1024 : 2048) && !(fp64 && all && wg > 512 && wg < 1024);
   if (wg <= (fp64 ? 448 : 512)) return true;
   if (set == HOPS_FACE || g.Vb < SITES) return false;
-  if (fp64) return all ? !b256 && wg >= 2048 && wg <= 16384 : wg <= 3072;
+  if (fp64) return all ? !b256 && wg >= 1024 && wg <= 16384 : wg <= 3072;
   if (all) return b256 ? wg <= 1792 : wg >= 1024 && wg <= (nl == 12 ? 2592 : 4096);
   return !b256 && wg <= (nl == 12 ? 768 : 2048);
 }
