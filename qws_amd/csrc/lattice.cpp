@@ -948,8 +948,9 @@ int Lattice::bicgstab_eo(double* x, const double* b, int maxiter, double tol, in
   // but scratch: the GPU does not wait for the host (8^4: 26 iterations 2.02 -> 1.63 ms).  Where
   // it may not be needed it waits instead: in the first half-step (a solve that is done then,
   // waiting / with the operator ahead: 16^4 92 / 126 us, 24^3 48 0.76 / 1.03 ms) and, where it takes
-  // longer than the wait (15 us on 16^4), within a factor of 10 of tol (a half-step gains 1.2
-  // to 3; a solve of 24^3 48 to 1e-8 with the wait / without: 18.4 / 18.8 ms).
+  // longer than the wait (15 us on 16^4), within a factor of tol (a half-step gains 1.2 to 3): to
+  // 1e-8 ahead always / but for a factor of 2 / of 10, 8 16^2 40 2.70 / 2.65 / 2.69 ms, 16^2 24^2
+  // 4.77 / 4.70 / 4.64, 24^3 48 18.7 / 18.5 / 18.4.
   if (!eo_ev_) QWS_HIP(hipEventCreateWithFlags(&eo_ev_, hipEventDisableTiming));
   auto ask = [&] {
     QWS_HIP(hipMemcpyAsync(sc_host_, sc_eo_, sizeof(Scalars), hipMemcpyDeviceToHost, st_));
@@ -970,7 +971,7 @@ int Lattice::bicgstab_eo(double* x, const double* b, int maxiter, double tol, in
   };
   int iter;
   double res = 0;  // as last seen
-  const double margin = g_.V <= 1 << 16 ? 1 : 10;
+  const double margin = g_.V <= 1 << 16 ? 1 : g_.V <= 1 << 17 ? 2 : 10;
   if (maxiter > 1) mt(q, p, DEO_DOT);
   for (iter = 1; iter < maxiter; ++iter) {
     launch_finalize(B, dpart, 2, sc_eo_, FIN_ALPHA, st_, groups);

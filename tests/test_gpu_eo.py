@@ -216,7 +216,7 @@ def test_eo_bicgstab_stops_at_either_half_step(L):
 @pytest.mark.parametrize("L", [[8, 4, 4, 8], [12, 16, 12, 32], [24, 24, 24, 20]])
 def test_eo_bicgstab_where_the_next_operator_waits(L):
     """Solves that start near their solution, or end soon after: done in the first half-step
-    or in one within a factor of 10 of tol, whose next operator waits for the check, x being
+    or in one that comes close to tol, whose next operator waits for the check, x being
     updated at once or (above 2^18 sites) at the end.  The largest lattice's operator (292 MB)
     goes past the caches, its sums with it.  True residual as above."""
     lat = Q.Lattice(L, [L[0] // 2] + L[1:], -1, 18, kappa=0.115)
